@@ -528,8 +528,7 @@ ER_DEV void gemv_q8_0_i8_fused_core(const uint8_t *const (&rowp)[R], void *const
             if (threadIdx.x + NT * (uint32_t)c < C16)
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    ss += xr[c][q].x * xr[c][q].x + xr[c][q].y * xr[c][q].y + xr[c][q].z * xr[c][q].z +
-                          xr[c][q].w * xr[c][q].w;
+                    ss = xl_add_sq(ss, xr[c][q]);
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
         if (lane == 0) red[wave] = ss;
@@ -1563,8 +1562,7 @@ ER_DEV void gemv_cuk_rows(const Rows &rows, const float *__restrict__ x, uint32_
                     for (int q = 0; q < VPL / 4; ++q) {
                         float4 &v = xr[p][q];
                         const float4 w = nw[p][q];
-                        const float sq = v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
-                        ssq += own ? sq : 0.0f;
+                        ssq += own ? xl_sq(v) : 0.0f;
                         v = float4{v.x * w.x, v.y * w.y, v.z * w.z, v.w * w.w};
                     }
                 }
@@ -1589,7 +1587,11 @@ ER_DEV void gemv_cuk_rows(const Rows &rows, const float *__restrict__ x, uint32_
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < J; ++j) {
-            float acc = F::dot(wb[j % D], xs, -0.0f, M0F);  // -0 + v == v: the add folds away
+            // Q4_K, Q8_0: -0 + v == v, the add folds away.  Q6_K starts from +0:
+            // its last step d * v + (-0) would fold to a product that the lane
+            // sum's first add then takes into an fma, on each lane its own of
+            // the pair, and the row sum would depend on the lane it is parked in
+            float acc = F::dot(wb[j % D], xs, F::FMT == ER_FMT_Q6_K ? 0.0f : -0.0f, M0F);
             __builtin_amdgcn_sched_barrier(0);
             if (j + D < J) issue((uint32_t)(j + D), j % D);
             __builtin_amdgcn_sched_barrier(0);
@@ -1725,10 +1727,11 @@ struct CukQ8Multi {
         const uint32_t m = seg(r, l);
         return pick3(m, W0, W1, W2) + (size_t)l * rowBytes;
     }
-    __device__ __forceinline__ void store(uint32_t r, float v) const {
+    __device__ __forceinline__ void store(uint32_t r, float v) const { store_at(r, blockIdx.y, v); }
+    __device__ __forceinline__ void store_at(uint32_t r, uint32_t t, float v) const {
         uint32_t l;
         const uint32_t m = seg(r, l);
-        const size_t out = (size_t)blockIdx.y * pick3(m, M0, M1, M2) + l;
+        const size_t out = (size_t)t * pick3(m, M0, M1, M2) + l;
         const float *rp = pick3(m, r0, r1, r2);
         void *yp = pick3(m, y0, y1, y2);
         const float o = rp ? v + rp[out] : v;

@@ -54,3 +54,26 @@
 // K-sliced CU-resident Q4_K / Q8_0 kernels for 8192 < K <= 16384 (gemv_cuk):
 // one kernel per row-step count 1..ER_CUK_MAX_STEPS (2 rows per step).
 #define ER_CUK_MAX_STEPS 16
+
+// Token-batched kernels (er_gemv_tok.hip): the order in which a row's slots are
+// added (that of the one-token kernel its M and K select) and the launch's
+// split of it, passed by value.
+#include <stdint.h>
+struct TokOrder {
+    uint32_t lpr;  // whole-row kernels: lanes per row (the tree's leaves)
+    uint32_t ns;   // ... and slots per lane (a leaf's chain); 0: K-sliced
+    uint32_t spw;  // K-sliced kernels: slots per slice (one tree each)
+    uint32_t upt;  // ... and 256-weight units a tree can touch
+    uint32_t kw;   // slices of K over the workgroup's waves: 1, 2, 4 or 8
+    uint32_t ups;  // units per slice (at most)
+    uint32_t lupp;  // log2 of the units per slice held in LDS at once (kw << lupp a multiple of 4)
+    uint32_t mg;   // i / ns or i / upt of a unit index i as i * mg >> 16
+    uint32_t part; // bytes of the partial row sums in LDS
+    uint32_t nfl;  // lanes per row of the fp32 re-evaluation
+};
+#define ER_TOK_MAX_UNITS 192  // kw * ups: 128 for whole rows (lpr ns / 4), 8 * 9 for K-sliced ones
+// X(RT, TG, 4 TG): 16 RT rows per wave, 4 TG tokens
+#define ER_TOK_CONFIGS(X) X(1, 1, 4) X(4, 1, 4) X(1, 2, 8) X(4, 2, 8) X(1, 4, 16) X(2, 4, 16)
+// Q6_K and fused Q8_0 with several slots per leaf, Q8_0 with slices inside a
+// unit: X(4, 2, 8) spills
+#define ER_TOK_CONFIGS_SMALL(X) X(1, 1, 4) X(4, 1, 4) X(1, 2, 8) X(1, 4, 16) X(2, 4, 16)

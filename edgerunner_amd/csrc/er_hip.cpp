@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cstdarg>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -183,6 +184,27 @@ constexpr I8Cfg kI8Multi1Cfg[] = {ER_I8_MULTI1_CONFIGS(ER_I8_ROW)};
 #undef ER_I8_ROW
 constexpr int kI8Multi1Count = (int)(sizeof(kI8Multi1Cfg) / sizeof(kI8Multi1Cfg[0]));
 
+// Token-batched kernels {RT, TG} (er_gemv_cfg.h), by kind: the three formats'
+// plain rows, the fused Q8_0 rows and the fused Q8_0 gate/up pairs.
+struct TokCfg {
+    uint8_t rt, tg;
+};
+#define ER_TOK_ROW(RT, TG, TT) {RT, TG},
+constexpr TokCfg kTokCfg[] = {ER_TOK_CONFIGS(ER_TOK_ROW)};
+#undef ER_TOK_ROW
+constexpr int kTokCount = (int)(sizeof(kTokCfg) / sizeof(kTokCfg[0]));
+enum TokKind { TOK_Q4K, TOK_Q8, TOK_Q6K, TOK_Q8_MULTI, TOK_Q8_SILU, TOK_KINDS };
+constexpr const char *kTokKindNames[TOK_KINDS] = {"q4k", "q8_0", "q6k", "q8_0_multi", "q8_0_silu"};
+// modes of a launch: one slot per leaf, several (c), slices inside a unit (s)
+enum TokMode { TOK_PLAIN, TOK_CHAIN, TOK_SPLIT, TOK_MODES };
+constexpr const char *kTokModeTags[TOK_MODES] = {"", "c", "s"};
+constexpr bool tok_built(int kind, int mode, const TokCfg &c) {
+    const bool fits = !(c.rt == 4 && c.tg == 2);  // ER_TOK_CONFIGS_SMALL
+    if (kind == TOK_Q4K || mode == TOK_PLAIN) return true;
+    if (kind == TOK_Q6K) return mode == TOK_CHAIN && fits;
+    return (kind == TOK_Q8 && mode == TOK_CHAIN) || fits;
+}
+
 // Kernel argument block of er_gemv_q4k_multi_* (matches Q4Multi in er_gemv.hip).
 struct Q4MultiArgs {
     const void *W[3];
@@ -229,6 +251,9 @@ struct er_hip_ctx {
     hipFunction_t fnQ8Silu[kI8MultiCount] = {};
     hipFunction_t fnQ4KMulti1[kI8Multi1Count] = {};  // one row computation per lane group
     hipFunction_t fnQ8Multi1[kI8Multi1Count] = {};
+    hipFunction_t fnTok[TOK_KINDS][TOK_MODES][kTokCount] = {};
+    int tok_mode = -1;  // ER_HIP_GEMV_TOK: 0 never, 1 whenever it applies, rt:tt:kw (2): with this split where it can
+    uint32_t tok_rt = 0, tok_tt = 0, tok_kw = 0;
     int cu_count = 0;
     int i8_override = -1;  // ER_HIP_GEMV_CONFIG=lpr:ns:r (benchmark sweeps only)
     int multi_override = -1;  // ER_HIP_GEMV_MULTI_CONFIG=lpr:ns:r for the multi-matrix kernels (tests, sweeps)
@@ -607,6 +632,133 @@ bool plan_cuk(const er_hip_ctx *ctx, Fmt f, uint32_t M, uint32_t K, uint32_t bat
     return true;
 }
 
+// Addition order of a row under the one-token kernel that M and K select
+// (TokOrder, without the launch's split): K-sliced trees or whole rows.
+TokOrder tok_order_cuk(const CukPlan &kp, Fmt f, uint32_t K) {
+    const uint32_t S = K / 64u;
+    TokOrder o{};
+    o.spw = f == Fmt::Q6_K ? 4u * ((S + 31u) / 32u) : (S + ER_CU_WAVES - 1u) / ER_CU_WAVES;
+    for (uint32_t s0 = 0; s0 < S; s0 += o.spw) {
+        const uint32_t s1 = std::min(s0 + o.spw, S);
+        o.upt = std::max(o.upt, (s1 + 3u) / 4u - s0 / 4u);
+    }
+    o.nfl = 64u / (2u << kp.pi);
+    return o;
+}
+TokOrder tok_order_rows(uint32_t lpr, uint32_t ns) {
+    TokOrder o{};
+    o.lpr = o.nfl = lpr;
+    o.ns = ns;
+    return o;
+}
+bool tok_order(const er_hip_ctx *ctx, Fmt f, uint32_t M, uint32_t K, TokOrder &o) {
+    CukPlan kp;
+    if (plan_cuk(ctx, f, M, K, 1u, kp)) {
+        o = tok_order_cuk(kp, f, K);
+        return true;
+    }
+    CuPlan cp;
+    if (plan_cu(ctx, f, M, K, 1u, cp)) {
+        const CuCfg &c = (f == Fmt::Q4_K ? kCuCfgQ4K : (f == Fmt::Q8_0 ? kCuCfgQ8 : kCuCfgQ6K))[cp.ci];
+        o = tok_order_rows(c.lpr, c.ns);
+        return true;
+    }
+    const int ci = pick_i8(K / 64u, M, ctx->cu_count, 1u);
+    if (ci < 0) return false;
+    o = tok_order_rows(kI8Cfg[ci].lpr, kI8Cfg[ci].ns);
+    return true;
+}
+
+// Split of a token-batched launch (er_gemv_tok.hip): configuration {RT, TG}
+// and slices of K kw, for `rows` rows of K weights and T tokens in order o.
+struct TokPlan {
+    int ci = -1, mode = 0;
+    TokOrder o{};
+    uint32_t grid = 0, lds = 0;
+};
+bool plan_tok(const er_hip_ctx *ctx, int kind, uint32_t rows, uint32_t K, uint32_t T, TokOrder o, TokPlan &p) {
+    const bool q6 = kind == TOK_Q6K, q4 = kind == TOK_Q4K;
+    const uint32_t S = K / 64u, cu = (uint32_t)ctx->cu_count;
+    const int mode = o.ns > 1u ? TOK_CHAIN : (o.ns == 0u && o.spw % 4u != 0u ? TOK_SPLIT : TOK_PLAIN);
+    // vector instructions of a 64-weight slot per row tile, and per tile and 4
+    // tokens (Q8_0 and Q6_K with the waits that their larger stages add)
+    const double perTile = q4 ? 16.0 : (q6 ? 50.0 : 28.0), perTok = q4 ? 17.0 : (q6 ? 34.0 : 21.0);
+    const double rowBytes = (double)K * (q4 ? 0.5625 : (q6 ? 0.8203125 : 1.0625));
+    double best = 0.0;
+    for (int ci = 0; ci < kTokCount; ++ci) {
+        const TokCfg &c = kTokCfg[ci];
+        if (!tok_built(kind, mode, c)) continue;
+        const uint32_t TT = 4u * c.tg, fac = q6 ? 96u : 64u;
+        const uint32_t nTok = (T + TT - 1u) / TT;
+        for (uint32_t kw = 1; kw <= 8u; kw *= 2u) {
+            TokOrder t = o;
+            t.kw = kw;
+            if (t.ns) {
+                const uint32_t leaves = t.lpr / kw;
+                if (leaves < 4u || leaves > 32u) continue;
+                t.ups = (std::min(leaves, S) + 3u) / 4u * t.ns;
+            } else {
+                t.ups = 8u / kw * t.upt;
+            }
+            if (kw * t.ups > ER_TOK_MAX_UNITS) continue;
+            t.mg = 65535u / (t.ns ? t.ns : t.upt) + 1u;
+            const uint32_t rowsWg = 16u * c.rt * (ER_CU_WAVES / kw);
+            const uint32_t nPart = t.ns || kw == 1u ? kw : 8u;
+            t.part = nPart * TT * rowsWg * 4u;
+            // limbs and factors of a phase, partial sums, the waves' stages
+            const uint32_t fixed = t.part + ER_CU_WAVES * std::min<uint32_t>(c.rt, 2u) * 16u * (q4 ? 144u : (q6 ? 224u : 272u));
+            // as many units per phase as fit: one workgroup per CU, or, where
+            // the kernel's registers allow two, half the LDS each
+            const uint32_t unit = TT * (768u + fac);
+            const uint64_t room = (c.rt == 1u ? ctx->info.lds_per_workgroup / 2u : ctx->info.lds_per_workgroup) - 4096u;
+            uint32_t lupp = kw >= 4u ? 0u : (kw == 2u ? 1u : 2u);
+            if ((uint64_t)(kw << lupp) * unit + fixed > ctx->info.lds_per_workgroup - 4096u) continue;
+            while ((1u << lupp) < t.ups && (uint64_t)(kw << (lupp + 1u)) * unit + fixed <= room) ++lupp;
+            t.lupp = lupp;
+            const uint32_t blocks = (rows + rowsWg - 1u) / rowsWg;
+            const uint64_t wgs = (uint64_t)blocks * nTok, grid = (uint64_t)((blocks + 7u) / 8u) * 8u * nTok;
+            if (grid > 0x7fffffffull) continue;
+            // microseconds of a launch, fitted to sweeps over the configurations
+            // (14336 x 4096, 4096 x 14336 and 1024 x 1024, 4 to 77 tokens; most
+            // within 15%): vector time at 2.1 GHz of a workgroup's walk (two
+            // waves per SIMD) and of its conversion of x (a pass of 170
+            // instructions per 1024 values), a latency per unit, the weight
+            // bytes, and a start per workgroup and launch
+            const double walk = t.ups * 4.0 * c.rt * (perTile + perTok * c.tg) * 8.0 / 2100.0;
+            // (under RMSNorm the sum of squares and the norm weights as well)
+            const bool norm = kind == TOK_Q8_MULTI || kind == TOK_Q8_SILU;
+            const double conv = std::min(TT, T) * (K / 1024.0) * (170.0 / 2100.0 + (norm ? 0.2 : 0.0));
+            const double res = c.rt == 1u && wgs > cu ? 2.0 : 1.0;  // workgroups sharing a CU
+            const double rounds = std::ceil((double)wgs / (cu * res));
+            const double cost = 3.0 + rounds * (1.5 + 0.4 * t.ups + res * (walk + conv + rowsWg * rowBytes / 45000.0));
+            if (ctx->tok_mode == 2 && (c.rt != ctx->tok_rt || TT != ctx->tok_tt || kw != ctx->tok_kw)) continue;
+            if (p.ci < 0 || cost < best) {
+                best = cost;
+                p.ci = ci;
+                p.mode = mode;
+                p.o = t;
+                p.grid = (uint32_t)grid;
+                p.lds = (kw << lupp) * unit + fixed;
+            }
+        }
+    }
+    // the one-token kernels over the tokens: a launch, then every token's
+    // weights again (from the Infinity Cache: 3.2 / 7.3 / 4.4 us per token of
+    // Q4_K / Q8_0 / Q6_K 14336 x 4096).  Few tokens and short matrices stay
+    // with them.
+    const double perTok1 = 0.08 + (double)rows * K * (q4 ? 6.2e-8 : (q6 ? 9.0e-8 : 8.5e-8));
+    if (ctx->tok_mode < 0 && best >= 3.0 + T * perTok1) return false;
+    return p.ci >= 0;
+}
+
+// Whether calls of two and more tokens take the token-batched kernels: rows of
+// whole 256-weight units that the integer kernels cover, no kernel forced.
+bool tok_applies(const er_hip_ctx *ctx, uint32_t K, uint32_t T) {
+    return T >= 2u && K % 256u == 0 && K <= kI8MaxK && ctx->gemv_fp32 == 0 && ctx->i8_override < 0 &&
+           ctx->multi_override < 0 && ctx->multi1_override < 0 && ctx->cu_mode < 0 && ctx->cuk_mode < 0 &&
+           ctx->tok_mode != 0;
+}
+
 er_status encode_gemv(er_hip_ctx *ctx, er_stream stream, Fmt f, er_buffer W, er_buffer x,
                       er_buffer y, uint32_t batch, uint32_t M, uint32_t K) {
     // shape validation first (it needs no device), then the context
@@ -621,6 +773,16 @@ er_status encode_gemv(er_hip_ctx *ctx, er_stream stream, Fmt f, er_buffer W, er_
 
     void *args[] = {&W.data, &x.data, &y.data, &M, &K};
     const bool q8Aligned = f == Fmt::Q8_0 && K % 64u == 0;
+    if (tok_applies(ctx, K, batch)) {
+        const int kind = f == Fmt::Q4_K ? TOK_Q4K : (f == Fmt::Q8_0 ? TOK_Q8 : TOK_Q6K);
+        TokOrder o;
+        TokPlan tp;
+        if (tok_order(ctx, f, M, K, o) && plan_tok(ctx, kind, M, K, batch, o, tp)) {
+            void *targs[] = {&W.data, &x.data, &y.data, &M, &K, &batch, &tp.o};
+            return launch_fn(ctx->fnTok[kind][tp.mode][tp.ci], "er_gemv_tok", dim3(tp.grid, 1, 1),
+                             dim3(64u * ER_CU_WAVES, 1, 1), tp.lds, stream, targs);
+        }
+    }
     CukPlan kp;
     if (plan_cuk(ctx, f, M, K, batch, kp)) {
         dim3 grid((M + kp.rowsPerWg - 1u) / kp.rowsPerWg, batch, 1);
@@ -1201,6 +1363,21 @@ struct Q8FusedSpec {
     bool silu;          // gate/up pairs, output silu(gate) * up
 };
 
+Q8MultiArgs q8_multi_args(const Q8FusedSpec &f) {
+    Q8MultiArgs a{};
+    for (int m = 0; m < 3; ++m) {
+        const int j = m < f.count ? m : 0;
+        a.W[m] = f.W[j].data;
+        a.y[m] = f.y[j].data;
+        a.res[m] = m < f.count ? (const float *)f.res[m].data : nullptr;
+        a.M[m] = m < f.count ? f.M[m] : 0u;
+    }
+    a.halfMask = f.halfMask;
+    a.normW = (const float *)f.normW.data;
+    a.eps = f.eps;
+    return a;
+}
+
 er_status encode_q8_fused(er_hip_ctx *ctx, er_stream stream, const Q8FusedSpec &f, er_buffer x,
                           uint32_t tokens, uint32_t K) {
     if (K == 0 || K % 32u != 0)
@@ -1260,6 +1437,38 @@ er_status encode_q8_fused(er_hip_ctx *ctx, er_stream stream, const Q8FusedSpec &
     // 14336 x 4096 28.00 -> 24.27.
     CukPlan kp;
     const uint64_t rowsV = f.silu ? 2u * Mt : Mt;
+    if (!anyK && tok_applies(ctx, K, tokens) && rowsV <= 0x7fffffffull) {
+        const int kind = f.silu ? TOK_Q8_SILU : TOK_Q8_MULTI;
+        TokOrder o;
+        TokPlan tp;
+        bool ok = false;
+        if (fused_on_cuk(ctx, rowsV, K) && plan_cuk(ctx, Fmt::Q8_0, (uint32_t)rowsV, K, 1u, kp, true)) {
+            o = tok_order_cuk(kp, Fmt::Q8_0, K);
+            ok = true;
+        } else {
+            const MultiPick mp = pick_multi(ctx, S, (uint32_t)rowsV, !f.silu, 1u);
+            if (mp.ci >= 0 || mp.ci1 >= 0) {
+                const I8Cfg &c = mp.ci >= 0 ? kI8MultiCfg[mp.ci] : kI8Multi1Cfg[mp.ci1];
+                o = tok_order_rows(c.lpr, c.ns);
+                ok = true;
+            }
+        }
+        if (ok && plan_tok(ctx, kind, (uint32_t)rowsV, K, tokens, o, tp)) {
+            const dim3 grid(tp.grid, 1, 1), block(64u * ER_CU_WAVES, 1, 1);
+            hipFunction_t fn = ctx->fnTok[kind][tp.mode][tp.ci];
+            if (f.silu) {
+                const float *normW = (const float *)f.normW.data;
+                float eps = f.eps;
+                uint32_t M = f.M[0];
+                void *args[] = {(void *)&f.W[0].data, (void *)&f.W[1].data, &x.data, (void *)&f.y[0].data,
+                                &normW, &eps, &M, &K, &tokens, &tp.o};
+                return launch_fn(fn, "er_gemv_q8_0_silu_tok", grid, block, tp.lds, stream, args);
+            }
+            Q8MultiArgs a = q8_multi_args(f);
+            void *args[] = {&a, &x.data, &K, &tokens, &tp.o};
+            return launch_fn(fn, "er_gemv_q8_0_multi_tok", grid, block, tp.lds, stream, args);
+        }
+    }
     if (!anyK && fused_on_cuk(ctx, rowsV, K) && plan_cuk(ctx, Fmt::Q8_0, (uint32_t)rowsV, K, tokens, kp, true)) {
         const uint32_t lds = xl_lds_bytes(K);
         dim3 grid((uint32_t)((rowsV + kp.rowsPerWg - 1u) / kp.rowsPerWg), tokens, 1);
@@ -1272,34 +1481,14 @@ er_status encode_q8_fused(er_hip_ctx *ctx, er_stream stream, const Q8FusedSpec &
             return launch_fn(ctx->fnQ8CukSilu[kp.pi][kp.j - 1], "er_gemv_q8_0_silu_cuk", grid,
                              dim3(64u * ER_CU_WAVES, 1, 1), lds, stream, args);
         }
-        Q8MultiArgs a{};
-        for (int m = 0; m < 3; ++m) {
-            const int j = m < f.count ? m : 0;
-            a.W[m] = f.W[j].data;
-            a.y[m] = f.y[j].data;
-            a.res[m] = m < f.count ? (const float *)f.res[m].data : nullptr;
-            a.M[m] = m < f.count ? f.M[m] : 0u;
-        }
-        a.halfMask = f.halfMask;
-        a.normW = normW;
-        a.eps = eps;
+        Q8MultiArgs a = q8_multi_args(f);
         void *args[] = {&a, &x.data, &K};
         return launch_fn(ctx->fnQ8CukMulti[kp.pi][kp.j - 1], "er_gemv_q8_0_multi_cuk", grid,
                          dim3(64u * ER_CU_WAVES, 1, 1), lds, stream, args);
     }
     const MultiPick mp = anyK ? MultiPick{} : pick_multi(ctx, S, (uint32_t)(f.silu ? 2u * Mt : Mt), !f.silu, tokens);
     if (mp.ci < 0 && mp.ci1 < 0) {
-        Q8MultiArgs a{};
-        for (int m = 0; m < 3; ++m) {
-            const int j = m < f.count ? m : 0;
-            a.W[m] = f.W[j].data;
-            a.y[m] = f.y[j].data;
-            a.res[m] = m < f.count ? (const float *)f.res[m].data : nullptr;
-            a.M[m] = m < f.count ? f.M[m] : 0u;
-        }
-        a.halfMask = f.halfMask;
-        a.normW = (const float *)f.normW.data;
-        a.eps = f.eps;
+        Q8MultiArgs a = q8_multi_args(f);
         // 2 rows (or 2 gate/up pairs) per wave
         const uint32_t rowsPerBlock = ER_GEMV_WAVES * 2u;
         void *args[] = {&a, &x.data, &K};
@@ -1321,17 +1510,7 @@ er_status encode_q8_fused(er_hip_ctx *ctx, er_stream stream, const Q8FusedSpec &
         return launch_fn(ctx->fnQ8Silu[ci], "er_gemv_q8_0_silu", grid, dim3(kGemvThreads, 1, 1), lds, stream,
                          args);
     }
-    Q8MultiArgs a{};
-    for (int m = 0; m < 3; ++m) {
-        const int j = m < f.count ? m : 0;
-        a.W[m] = f.W[j].data;
-        a.y[m] = f.y[j].data;
-        a.res[m] = m < f.count ? (const float *)f.res[m].data : nullptr;
-        a.M[m] = m < f.count ? f.M[m] : 0u;
-    }
-    a.halfMask = f.halfMask;
-    a.normW = normW;
-    a.eps = eps;
+    Q8MultiArgs a = q8_multi_args(f);
     const uint32_t rowsPerBlock = ER_GEMV_WAVES * (64u / c.lpr) * c.r;
     void *args[] = {&a, &x.data, &K};
     dim3 grid((uint32_t)((Mt + rowsPerBlock - 1) / rowsPerBlock), tokens, 1);
@@ -1556,6 +1735,31 @@ er_status er_hip_create(int device, er_hip_ctx **out_ctx) {
                 delete ctx;
                 return fail(ER_ERR_FUNCTION_NOT_FOUND, "functionNotFound(%s): %s", name, hipGetErrorString(e));
             }
+        }
+    }
+    for (int kind = 0; kind < TOK_KINDS; ++kind)
+        for (int mode = 0; mode < TOK_MODES; ++mode)
+            for (int i = 0; i < kTokCount; ++i) {
+                if (!tok_built(kind, mode, kTokCfg[i])) continue;
+                char name[64];
+                std::snprintf(name, sizeof(name), "er_gemv_%s_tok%s_r%u_t%u", kTokKindNames[kind], kTokModeTags[mode],
+                              (unsigned)kTokCfg[i].rt, 4u * (unsigned)kTokCfg[i].tg);
+                e = hipModuleGetFunction(&ctx->fnTok[kind][mode][i], ctx->module, name);
+                if (e != hipSuccess) {
+                    (void)hipModuleUnload(ctx->module);
+                    delete ctx;
+                    return fail(ER_ERR_FUNCTION_NOT_FOUND, "functionNotFound(%s): %s", name, hipGetErrorString(e));
+                }
+            }
+    if (const char *tv = std::getenv("ER_HIP_GEMV_TOK")) {
+        unsigned a = 0, b = 0, c = 0;
+        if (std::sscanf(tv, "%u:%u:%u", &a, &b, &c) == 3) {
+            ctx->tok_mode = 2;
+            ctx->tok_rt = a;
+            ctx->tok_tt = b;
+            ctx->tok_kw = c;
+        } else {
+            ctx->tok_mode = std::atoi(tv) != 0 ? 1 : 0;
         }
     }
     if (const char *gv = std::getenv("ER_HIP_GEMM_VARIANT")) ctx->gemm_variant = std::atoi(gv);

@@ -5,6 +5,7 @@
 // plus probes and clock-stamped GEMM copies).
 #include "er_dequant.hip"
 #include "er_gemv.hip"
+#include "er_gemv_tok.hip"
 #include "er_gemm.hip"
 #include "er_quant.hip"
 #include "er_scratch.hip"

@@ -144,6 +144,15 @@ ER_DEV float xl_group_sum8(float r) {
 }
 
 
+// x^2 terms of the RMSNorm sums: one float4's squares, and added to ss.  The
+// fused multiply-adds are written out: left to the compiler, which product of
+// a sum of two becomes the fused one may differ between kernels, and with it
+// the last bit of the factor.
+ER_DEV float xl_sq(const float4 &v) {
+    return __builtin_fmaf(v.w, v.w, __builtin_fmaf(v.z, v.z, __builtin_fmaf(v.y, v.y, v.x * v.x)));
+}
+ER_DEV float xl_add_sq(float ss, const float4 &v) { return ss + xl_sq(v); }
+
 // Loads of chunk c (16 values) of x for thread `tid`; XG chunks per thread.
 // Out-of-range chunks reload the last chunk (always in bounds, never stored).
 template <int XG, int NT>
@@ -173,19 +182,15 @@ ER_DEV void xl_scale(float mx, float *sg, float *inv) {
     *inv = live ? __uint_as_float((254u - (b >> 23)) << 23) : 0.0f;
 }
 
-// Converts one 16-value chunk (index tRaw, values in xr) into LDS.  The 4
-// chunks of a 64-group are held by 4 consecutive lanes, which exchange their
-// maxima; every lane of the wave must call this together.
-ER_DEV void xl_store_chunk(uint32_t *lds, uint32_t K, const float4 (&xr)[4], uint32_t tRaw, XlCheck *ck = nullptr) {
-    const uint32_t C16 = K >> 4;
-    float v[16];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        v[4 * q + 0] = xr[q].x;
-        v[4 * q + 1] = xr[q].y;
-        v[4 * q + 2] = xr[q].z;
-        v[4 * q + 3] = xr[q].w;
-    }
+// One 16-value chunk converted: limb bytes lb[plane][values 4d .. 4d + 3], the
+// chunk sum, and its 64-group's scale and rest energy.  The 4 chunks of a
+// 64-group are held by 4 consecutive lanes, which exchange their maxima; every
+// lane of the wave must convert together.
+struct XlChunk {
+    uint32_t lb[ER_XL_PLANES][4];
+    float sum, sg, rest;
+};
+ER_DEV void xl_chunk(const float (&v)[16], XlChunk &o) {
     float mx = 0.0f, sa = 0.0f, sb = 0.0f;
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
@@ -197,35 +202,51 @@ ER_DEV void xl_store_chunk(uint32_t *lds, uint32_t K, const float4 (&xr)[4], uin
         mx = fmaxf(mx, fabsf(v[q]));
         sb += v[q];
     }
-    const float sm = sa + sb;
+    o.sum = sa + sb;
     const float lmx = mx;
     mx = dpp_max_nonneg<ER_DPP_QUAD_XOR1>(mx);
     mx = dpp_max_nonneg<ER_DPP_QUAD_XOR2>(mx);
-    float sg, inv;
-    xl_scale(mx, &sg, &inv);
-    const float rest = xl_rest_energy(v, lmx, mx, xl_group_sum4);
+    float inv;
+    xl_scale(mx, &o.sg, &inv);
+    o.rest = xl_rest_energy(v, lmx, mx, xl_group_sum4);
     // digits of u = xi + C are bytes 0..2 of fma(v, 1/s_g, 2^23 + C)
     uint32_t u[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) u[q] = __float_as_uint(__builtin_fmaf(v[q], inv, ER_XL_MAGIC));
-    uint32_t lb[ER_XL_PLANES][4];
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
         const uint32_t a = u[4 * d], b = u[4 * d + 1], c = u[4 * d + 2], e = u[4 * d + 3];
-        // byte k of the result = byte `sel` of values a, b, c, e
+        // 4 x 3 byte transpose: bytes 0, 1 of a, b and of c, e, then byte 2
+        const uint32_t ab = __builtin_amdgcn_perm(b, a, 0x05010400u), ce = __builtin_amdgcn_perm(e, c, 0x05010400u);
+        const uint32_t d2 = __builtin_amdgcn_perm(ce, ab, 0x05040100u);
+        const uint32_t d1 = __builtin_amdgcn_perm(ce, ab, 0x07060302u);
         const uint32_t d0 = __builtin_amdgcn_perm(__builtin_amdgcn_perm(e, c, 0x0c0c0602u),
                                                   __builtin_amdgcn_perm(b, a, 0x0c0c0602u), 0x05040100u);
-        const uint32_t d1 = __builtin_amdgcn_perm(__builtin_amdgcn_perm(e, c, 0x0c0c0501u),
-                                                  __builtin_amdgcn_perm(b, a, 0x0c0c0501u), 0x05040100u);
-        const uint32_t d2 = __builtin_amdgcn_perm(__builtin_amdgcn_perm(e, c, 0x0c0c0400u),
-                                                  __builtin_amdgcn_perm(b, a, 0x0c0c0400u), 0x05040100u);
         // d - 128 as int8 is d ^ 0x80; d0 - 64 (d0 < 128) is d0 ^ 0x40 with bit 7
         // set where bit 6 of d0 ^ 0x40 is set (sign extension of a 7-bit value)
         const uint32_t t = d0 ^ 0x40404040u;
-        lb[0][d] = t ^ ((t & 0x40404040u) << 1);
-        lb[1][d] = d1 ^ 0x80808080u;
-        lb[2][d] = d2 ^ 0x80808080u;
+        o.lb[0][d] = t ^ ((t & 0x40404040u) << 1);
+        o.lb[1][d] = d1 ^ 0x80808080u;
+        o.lb[2][d] = d2 ^ 0x80808080u;
     }
+}
+
+// Converts one 16-value chunk (index tRaw, values in xr) into LDS; as xl_chunk,
+// every lane of the wave must call this together.
+ER_DEV void xl_store_chunk(uint32_t *lds, uint32_t K, const float4 (&xr)[4], uint32_t tRaw, XlCheck *ck = nullptr) {
+    const uint32_t C16 = K >> 4;
+    float v[16];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        v[4 * q + 0] = xr[q].x;
+        v[4 * q + 1] = xr[q].y;
+        v[4 * q + 2] = xr[q].z;
+        v[4 * q + 3] = xr[q].w;
+    }
+    XlChunk o;
+    xl_chunk(v, o);
+    const float sm = o.sum, sg = o.sg, rest = o.rest;
+    const auto &lb = o.lb;
     if (ck) {
         const bool st = tRaw < C16, first = st && (tRaw & 3u) == 0;
         ck->e = __builtin_fmaf(first && rest > 0.0f ? sg : 0.0f, sg, ck->e);
@@ -279,12 +300,11 @@ ER_DEV void xl_store_half(uint32_t *lds, uint32_t K, const float4 (&xr)[2], uint
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
         const uint32_t a = u[4 * d], b = u[4 * d + 1], c = u[4 * d + 2], e = u[4 * d + 3];
+        const uint32_t ab = __builtin_amdgcn_perm(b, a, 0x05010400u), ce = __builtin_amdgcn_perm(e, c, 0x05010400u);
+        const uint32_t d2 = __builtin_amdgcn_perm(ce, ab, 0x05040100u);
+        const uint32_t d1 = __builtin_amdgcn_perm(ce, ab, 0x07060302u);
         const uint32_t d0 = __builtin_amdgcn_perm(__builtin_amdgcn_perm(e, c, 0x0c0c0602u),
                                                   __builtin_amdgcn_perm(b, a, 0x0c0c0602u), 0x05040100u);
-        const uint32_t d1 = __builtin_amdgcn_perm(__builtin_amdgcn_perm(e, c, 0x0c0c0501u),
-                                                  __builtin_amdgcn_perm(b, a, 0x0c0c0501u), 0x05040100u);
-        const uint32_t d2 = __builtin_amdgcn_perm(__builtin_amdgcn_perm(e, c, 0x0c0c0400u),
-                                                  __builtin_amdgcn_perm(b, a, 0x0c0c0400u), 0x05040100u);
         const uint32_t t = d0 ^ 0x40404040u;
         lb[0][d] = t ^ ((t & 0x40404040u) << 1);
         lb[1][d] = d1 ^ 0x80808080u;

@@ -1,0 +1,148 @@
+"""Token-batched GEMV kernels (two and more tokens): every row of every token
+equals the one-token call of the same matrix bit for bit, over the addition
+orders that M and K select (whole rows with one and several slots per lane,
+K-sliced rows whose slices start at and inside a 256-weight unit), row and
+token remainders, every compiled configuration and slice count, and x the
+limbs cannot carry.  The one-token calls are themselves held to the oracle
+(test_gpu_gemv.py, test_gpu_gemv_cuk.py, test_gpu_fused_q8.py)."""
+import os
+
+import numpy as np
+import pytest
+
+import edgerunner_amd.synth as synth
+from edgerunner_amd import Context, FusedQ8Kernel, GEMVKernel
+from oracle import ref
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+FMTS = ("q4_k", "q8_0", "q6_k")
+NAME = {"q4_k": "Q4K", "q6_k": "Q6K", "q8_0": "Q8_0"}
+
+
+def batched_and_single(ctx, fmt, W, x, M, K, T):
+    """(batched [T, M], the T one-token calls [T, M])."""
+    g = GEMVKernel(ctx)
+    wb, xb, yb, y1 = ctx.upload(W), ctx.upload(x), ctx.alloc(4 * T * M), ctx.alloc(4 * T * M)
+    try:
+        yb.upload(np.full(T * M, np.float32(7e30)))
+        getattr(g, f"encodeBatched{NAME[fmt]}Weights")(None, wb, xb, yb, T, M, K)
+        for t in range(T):
+            getattr(g, f"encode{NAME[fmt]}Weights")(None, wb, xb.view(4 * t * K, 4 * K), y1.view(4 * t * M, 4 * M), M, K)
+        ctx.synchronize()
+        return yb.download(np.float32).reshape(T, M), y1.download(np.float32).reshape(T, M)
+    finally:
+        for b in (wb, xb, yb, y1):
+            b.free()
+
+
+def forced(split):
+    """A context whose calls of two and more tokens take these kernels: "1" with
+    the planner's split, "rt:tt:kw" with this one where a shape allows it."""
+    old = os.environ.get("ER_HIP_GEMV_TOK")
+    os.environ["ER_HIP_GEMV_TOK"] = split
+    try:
+        return Context(0)
+    finally:
+        if old is None:
+            os.environ.pop("ER_HIP_GEMV_TOK", None)
+        else:
+            os.environ["ER_HIP_GEMV_TOK"] = old
+
+
+@pytest.fixture(scope="module")
+def tok():
+    c = forced("1")
+    yield c
+    c.close()
+
+
+# K: lane trees of 64 .. 4 leaves, several slots per lane (2560 and 3072 with
+# many rows), K-sliced rows (4096 Q4_K; 4352, 5120, 11008 start slices inside a
+# unit; 14336 and 16384 need several LDS phases)
+SHAPES = [(1, 256, 2), (17, 512, 3), (33, 1280, 9), (300, 1024, 5), (9000, 768, 4), (8192, 3072, 6), (10000, 2560, 3),
+          (2100, 4096, 17), (515, 4352, 7), (260, 5120, 16), (130, 11008, 5), (100, 14336, 19), (40, 16384, 33)]
+
+
+@pytest.mark.parametrize("M,K,T", SHAPES)
+@pytest.mark.parametrize("fmt", FMTS)
+def test_rows_equal_one_token_calls(tok, fmt, M, K, T):
+    W = synth.weights(fmt, synth.seed(96, 1), M, K)
+    x = synth.normal_f32(synth.seed(96, 2), T * K)
+    got, one = batched_and_single(tok, fmt, W, x, M, K, T)
+    assert np.array_equal(got, one)
+    rows = slice(0, min(M, 64))
+    n = len(W) // M
+    exp = np.stack([ref.gemv(fmt, W[:n * min(M, 64)], x[t * K:(t + 1) * K], min(M, 64), K) for t in (0, T - 1)])
+    assert rel_l2(got[[0, T - 1]][:, rows], exp) < 1e-3
+
+
+@pytest.mark.parametrize("rt,tt", [(1, 4), (4, 4), (1, 8), (4, 8), (1, 16), (2, 16)])
+def test_every_split(rt, tt):
+    """Each compiled {row tiles, tokens} with every count of K slices, plain
+    rows (K = 1024), chained slots (9000 x 768), split slices (K = 5120) and
+    several phases (K = 14336)."""
+    for kw in (1, 2, 4, 8):
+        c = forced(f"{rt}:{tt}:{kw}")
+        try:
+            for M, K, T in ((70, 1024, 5), (9000, 768, 2), (50, 5120, 6), (45, 14336, 18)):
+                for fmt in FMTS:
+                    W = synth.weights(fmt, synth.seed(96, 3), M, K)
+                    x = synth.normal_f32(synth.seed(96, 4), T * K)
+                    got, one = batched_and_single(c, fmt, W, x, M, K, T)
+                    assert np.array_equal(got, one), (kw, M, K, T, fmt)
+        finally:
+            c.close()
+
+
+@pytest.mark.parametrize("dim,q,kv,T", [(1024, 70, 30, 5), (2560, 5000, 1300, 3), (4096, 4096, 1024, 18),
+                                        (5120, 300, 77, 6), (14336, 130, 40, 9), (14336, 2100, 40, 2)])
+def test_fused_q8_rows_equal_one_token_calls(tok, dim, q, kv, T):
+    """RMSNorm + QKV (fp32 and fp16 V) and gate/up + SiLU."""
+    ctx = tok
+    f = FusedQ8Kernel(ctx)
+    W = [synth.q8_0(synth.seed(97, i), m, dim) for i, m in enumerate((q, kv, kv))]
+    x = synth.normal_f32(synth.seed(97, 5), T * dim)
+    nw = (np.float32(0.5) + np.abs(synth.normal_f32(synth.seed(97, 6), dim))).astype(np.float32)
+    b = [ctx.upload(a) for a in (*W, x, nw)]
+    sizes = (4 * q, 4 * kv, 2 * kv, 4 * kv, 4 * kv)  # q, k, v16, v32, act
+    outs = [ctx.alloc(T * n) for n in sizes]
+    one = [ctx.alloc(T * n) for n in sizes]
+
+    def encode(xb, o, n):
+        f.encodeFusedQKV(None, *b[:3], xb, o[0], o[1], o[2], b[4], q, kv, dim, n, 1e-5)
+        f.encodeFusedQKVTurbo(None, *b[:3], xb, o[0], o[1], o[3], b[4], q, kv, dim, n, 1e-5)
+        f.encodeFusedGateUpSilu(None, b[1], b[2], xb, o[4], b[4], kv, dim, n, 1e-5)
+    try:
+        encode(b[3], outs, T)
+        for t in range(T):
+            encode(b[3].view(4 * t * dim, 4 * dim), [o.view(t * n, n) for o, n in zip(one, sizes)], 1)
+        ctx.synchronize()
+        for o, w in zip(outs, one):
+            assert np.array_equal(o.download(np.uint8), w.download(np.uint8))
+    finally:
+        for buf in b + outs + one:
+            buf.free()
+
+
+@pytest.mark.parametrize("M,K", [(100, 1024), (2100, 4096), (60, 14336)])
+@pytest.mark.parametrize("fmt", FMTS)
+def test_x_the_limbs_cannot_carry(tok, fmt, M, K):
+    """A token with NaN, one with infinities and one whose outliers send the
+    launch to its fp32 evaluation.  All equal the one-token calls bit for bit
+    except the last: its rows are plain fp32 sums of K products, in which the
+    two kernels' compilers may or may not fuse multiply and add, each worth
+    up to 2^-24 of a partial sum per term (K 2^-24 = 1e-3 at most, sqrt(K)
+    2^-24 = 7e-6 for errors of random sign)."""
+    T = 6
+    W = synth.weights(fmt, synth.seed(98, 1), M, K)
+    x = synth.normal_f32(synth.seed(98, 2), T * K).reshape(T, K)
+    x[1, 5] = np.nan
+    x[2, K - 1], x[2, 70] = np.inf, -np.inf
+    x[4, ::64] = 1e6
+    got, one = batched_and_single(tok, fmt, W, x, M, K, T)
+    exact = [0, 1, 2, 3, 5]
+    assert np.array_equal(got[exact], one[exact], equal_nan=True)
+    assert rel_l2(got[4], one[4]) < 7e-6
+    assert np.isnan(got[1]).all() and np.isfinite(got[[0, 3, 4, 5]]).all()
