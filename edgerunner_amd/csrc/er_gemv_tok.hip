@@ -36,7 +36,7 @@
 // Measured, us a call, the one-token kernels over the tokens -> these (the
 // planner's choice; weights of several matrices in turn):
 //   tokens            5             16             32             77
-//   Q4_K 14336x4096   25.8 -> 20.2   57.5 -> 33.3  111.0 -> 47.4  254.6 -> 112
+//   Q4_K 14336x4096   25.8 -> 18.9   57.5 -> 33.3  111.0 -> 47.4  254.6 -> 112
 //   Q8_0 14336x4096   39.9 -> 26.4  117.7 -> 36.0  233.8 -> 50.4  559.7 -> 136
 //   Q6_K 4096x14336   40.3 -> 36.8  102.2 -> 58.0  201.7 -> 90.1  482.5 -> 228
 #include "er_gemv_cfg.h"
@@ -66,7 +66,7 @@ struct TokUnit {
 //   spw consecutive slots; slice ks holds trees [8 ks / KW, 8 (ks + 1) / KW).
 ER_DEV uint32_t tok_unit(const TokOrder &o, uint32_t S, uint32_t ks, uint32_t i) {
     if (o.ns) {
-        const uint32_t leaves = o.lpr / o.kw, n = i / o.ns, j = i - n * o.ns;
+        const uint32_t leaves = o.lpr >> __builtin_ctz(o.kw), n = (i * o.mg) >> 16, j = i - n * o.ns;
         const uint32_t l0 = ks * leaves + 4u * n;  // first leaf of the unit
         if (4u * n >= leaves || l0 >= S) return ER_TOK_NONE;
         const uint32_t slot = l0 + o.lpr * j;
@@ -76,7 +76,7 @@ ER_DEV uint32_t tok_unit(const TokOrder &o, uint32_t S, uint32_t ks, uint32_t i)
         const uint32_t pm = slot < S ? 15u : 0u;
         return (min(slot, S - 4u) >> 2) | pm << 8 | (4u * n + 4u) << 12 | ins << 20 | flush << 21 | live << 22;
     }
-    const uint32_t n = i / o.upt, k = i - n * o.upt, per = 8u / o.kw;
+    const uint32_t n = (i * o.mg) >> 16, k = i - n * o.upt, per = 8u >> __builtin_ctz(o.kw);
     if (n >= per) return ER_TOK_NONE;
     const uint32_t s0 = (ks * per + n) * o.spw, s1 = min(s0 + o.spw, S);
     if (s0 >= S) return ER_TOK_NONE;
@@ -483,10 +483,10 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
                      const TokOrder o) {
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     constexpr uint32_t TT = 4u * TG, NT = 64u * ER_CU_WAVES;
-    __shared__ uint32_t units[ER_TOK_MAX_UNITS];
+    __shared__ uint32_t units[ER_TOK_MAX_UNITS];  // slice ks, index i at ks * ups + i
     __shared__ float rmsv[TT];
     __shared__ float2 chk[NT / 32u];
-    __shared__ uint32_t nfv[TT], badv[TT], anyBad;
+    __shared__ uint32_t nfw[ER_CU_WAVES];  // [wave] tokens it saw a non-finite chunk sum of
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t S = K >> 6, kw = o.kw, rg = ER_CU_WAVES / kw, rowsWg = 16u * RT * rg;
     const uint32_t ks = wave % kw, grp = wave / kw;
@@ -497,7 +497,6 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
     if (blk * rowsWg >= M) return;
     const uint32_t nT = min(TT, T - t0);  // live tokens
     const uint32_t r = lane >> 4;         // quarter of the positions, and token of each group
-    const uint32_t total = kw * o.ups;    // units: slice ks, index i at ks * ups + i
 
     // x of a phase: a wave pass is one token's x of four units (one 16-value
     // chunk per lane); this wave makes passes wave, wave + 8, ...
@@ -531,22 +530,13 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
     load_x(0, wave, xr[0], wr[0]);
     __builtin_amdgcn_sched_barrier(0);
 
-    for (uint32_t i = tid; i < total; i += NT) {
-        const uint32_t sl = i / o.ups;
-        units[i] = tok_unit(o, S, sl, i - sl * o.ups);
-    }
-    if (tid < TT) nfv[tid] = 0u;
-    if (tid == 0) anyBad = 0u;
     if constexpr (Rows::NORM) {
         for (uint32_t t = wave; t < nT; t += ER_CU_WAVES) {
             const float ss = rows.normW ? tok_sum_sq(o, x + (size_t)(t0 + t) * K, K) : 0.0f;
             if (lane == 0) rmsv[t] = rows.normW ? 1.0f / __builtin_sqrtf(ss / (float)K + rows.eps) : 1.0f;
         }
+        __syncthreads();
     }
-    __syncthreads();
-    auto unit = [&](uint32_t i) {
-        return TokUnit{i < o.ups ? (uint32_t)__builtin_amdgcn_readfirstlane((int)units[ks * o.ups + i]) : ER_TOK_NONE};
-    };
     // this lane's granule of a slot's limbs: quarter r of limb lane % 4 (3: a
     // copy, its sums are not read) of token lane % 16 / 4.  A quarter's three
     // limbs lie side by side: 8 lanes of a read meet no bank twice
@@ -561,6 +551,7 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
     // slice of K, added up in order as they finish
     const uint32_t per = o.ns || kw == 1u ? 1u : 8u / kw, nPart = per * kw, stp = TT * rowsWg;
     float *part = (float *)(facs + (kw << o.lupp) * (TT * F::FAC));
+    uint32_t nfm = 0;  // tokens with a non-finite chunk sum
     auto convert = [&](uint32_t ps, const float4 (&xr)[4], const float4 (&wr)[NW]) {
         const uint32_t t = ps >> lq, v = 4u * (ps - (t << lq)) + r;
         float xv[16];
@@ -585,7 +576,7 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
         }
         XlChunk ck;
         xl_chunk(xv, ck);
-        if (__builtin_amdgcn_ballot_w64(!__builtin_isfinite(ck.sum)) != 0 && lane == 0) nfv[t] = 1u;
+        if (__builtin_amdgcn_ballot_w64(!__builtin_isfinite(ck.sum)) != 0) nfm |= 1u << t;
         // the chunk's slot, and the granules of its two 8-value pieces
         constexpr bool Q6 = F::FMT == ER_FMT_Q6_K;
         const uint32_t m = (c16 >> 1) & 3u;  // Q6_K granule
@@ -625,13 +616,25 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
         low[q] = F::FMT == ER_FMT_Q6_K ? (uint32_t)(uintptr_t)rows.row(min(row0 + 16u * q + (lane & 15u), M - 1u)) : 0u;
     }
     typename F::Ld ld[RT];
-    TokUnit cu = unit(0);
+    TokUnit cu{(uint32_t)__builtin_amdgcn_readfirstlane((int)tok_unit(o, S, ks, 0))};
     // the first pair's bytes leave before x is converted, the others after it
     // (an absent unit: super-block 0).  With all four tiles' loads ahead of it
     // the conversion began when they had left, 6 us into the launch.
 #pragma unroll
     for (int q = 0; q < PT; ++q) F::load(ld[q], rp[q], cu.sb(), lc);
     __builtin_amdgcn_sched_barrier(0);
+
+    // the units, for the walk: written behind the first loads and read after
+    // the conversion's barrier, so the table costs no barrier of its own (with
+    // one, and the rows summed through LDS at the end, a call took 0.3 to 0.8
+    // us more: Q4_K 4096 x 4096 x 5 10.3 -> 9.7 us, 14336 x 4096 x 5 19.4 ->
+    // 18.9, Q8_0 1024 x 1024 x 4 6.2 -> 5.3); formed on scalars at every unit
+    // instead, long slices lose it again (4096 x 14336 x 5 27.7 -> 28.6)
+    if (grp == 0)
+        for (uint32_t i = lane; i < o.ups; i += 64u) units[ks * o.ups + i] = tok_unit(o, S, ks, i);
+    auto unit = [&](uint32_t i) {
+        return TokUnit{i < o.ups ? (uint32_t)__builtin_amdgcn_readfirstlane((int)units[ks * o.ups + i]) : ER_TOK_NONE};
+    };
 
     // st: the addition tree as a binary counter, level l the sum of 2^l of its
     // steps (a unit's four leaves, or one leaf where slices start inside a
@@ -831,21 +834,27 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
     ce = group_sum<CW>(ce);
     cr = group_sum<CW>(cr);
     if (tid % CW == 0) chk[tid / CW] = float2{ce, cr};
+    if (lane == 0) nfw[wave] = nfm;
     __syncthreads();
-    if (tid < nT) {
-        float e = 0.0f, q = 0.0f;
+    // every wave decides for itself, so that rows with no such token are stored
+    // straight from their sums: bit t of ill (fp32 over every term), of
+    // nf (over the non-finite ones)
+    uint32_t nf = 0;
 #pragma unroll
-        for (uint32_t w = 0; w < CN; ++w) {
-            e += chk[tid * CN + w].x;
-            q += chk[tid * CN + w].y;
-        }
-        const bool ill = xl_ill_rule(e, q, F::FMT == ER_FMT_Q8_0 ? 1.0f : 4.0f);
-        badv[tid] = ill ? 2u : nfv[tid];
-        if (ill || nfv[tid]) anyBad = 1u;
+    for (uint32_t w = 0; w < ER_CU_WAVES; ++w) nf |= nfw[w];
+    float ee = 0.0f, rr = 0.0f;
+#pragma unroll
+    for (uint32_t w = 0; w < CN; ++w) {
+        const float2 c = chk[min(lane, TT - 1u) * CN + w];
+        ee += c.x;
+        rr += c.y;
     }
-    // row values: slices as the tree's top levels (whole rows) or in order
-    for (uint32_t i = tid; i < rowsWg * nT; i += NT) {
-        const uint32_t at = i;  // t rowsWg + row
+    const uint32_t ill = (uint32_t)__builtin_amdgcn_ballot_w64(lane < nT && xl_ill_rule(ee, rr, F::FMT == ER_FMT_Q8_0 ? 1.0f : 4.0f));
+    const uint32_t bad = (uint32_t)__builtin_amdgcn_readfirstlane((int)(ill | nf));
+    // row value (t, row) at part[t rowsWg + row]: slices as the tree's top
+    // levels (whole rows) or in order
+    const uint32_t lr = __builtin_ctz(rowsWg);
+    auto value = [&](uint32_t at) {
         float v;
         if (o.ns) {
             if (nPart == 1u) {
@@ -861,48 +870,54 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
         } else {
             v = 0.0f;
             for (uint32_t q = 0; q < nPart; ++q) v += part[at + q * stp];
-            if constexpr (Rows::NORM) v *= rmsv[i / rowsWg];
+            if constexpr (Rows::NORM) v *= rmsv[at >> lr];
         }
-        part[at] = v;  // only this thread reads slice 0 of (row, t)
-    }
-    __syncthreads();
-    if (anyBad) {
-        // tokens whose x the limbs do not carry (er_nonfinite.h, the
-        // conditioning rule of er_xlimbs.h): their rows again in fp32 from the
-        // raw weights, one row per lane group as the one-token kernels do
-        const uint32_t L = o.nfl, G = NT / L;
-        for (uint32_t i = tid / L; i < (rowsWg + G - 1u) / G * G; i += G) {
-            const uint32_t rw = min(blk * rowsWg + i, M - 1u), li = lane % L;
-            for (uint32_t t = 0; t < nT; ++t) {
-                if (!badv[t]) continue;
-                const float *xt = x + (size_t)(t0 + t) * K;
-                float sp[1] = {0.0f}, h = 0.0f;
-                nf_terms<1>([&](int, uint32_t k) { return weight_at<F::FMT>(end.row(rw), k); },
-                            [&](uint32_t k) {
-                                if constexpr (Rows::NORM)
-                                    return rows.normW ? xt[k] * rmsv[t] * rows.normW[k] : xt[k];
-                                else
-                                    return xt[k];
-                            },
-                            nullptr, K >> 4, li, L, sp, h, badv[t] == 2u);
-                const float v = tok_group_sum(sp[0], L), hs = tok_group_sum(h, L);
-                if (li == 0 && i < rowsWg && (badv[t] == 2u || hs > 0.0f)) part[t * rowsWg + i] = v;
+        return v;
+    };
+    auto store_rows = [&](auto val) {
+        if constexpr (Rows::PAIRS) {
+            for (uint32_t i = tid; i < (nT << (lr - 1u)); i += NT) {
+                const uint32_t t = i >> (lr - 1u), at = 2u * i, row = blk * rowsWg + (at & (rowsWg - 1u));
+                if (row < M) end.store(row, t0 + t, Rows::act(val(at)) * val(at + 1u));
+            }
+        } else {
+            for (uint32_t i = tid; i < (nT << lr); i += NT) {
+                const uint32_t row = blk * rowsWg + (i & (rowsWg - 1u));
+                if (row < M) end.store(row, t0 + (i >> lr), val(i));
             }
         }
-        __syncthreads();
+    };
+    if (bad == 0u) {
+        store_rows(value);
+        return;
     }
-    if constexpr (Rows::PAIRS) {
-        const uint32_t pairs = rowsWg / 2u;
-        for (uint32_t i = tid; i < pairs * nT; i += NT) {
-            const uint32_t t = i / pairs, rl = 2u * (i % pairs), row = blk * rowsWg + rl;
-            if (row < M) end.store(row, t0 + t, Rows::act(part[t * rowsWg + rl]) * part[t * rowsWg + rl + 1u]);
-        }
-    } else {
-        for (uint32_t i = tid; i < rowsWg * nT; i += NT) {
-            const uint32_t t = i / rowsWg, row = blk * rowsWg + i % rowsWg;
-            if (row < M) end.store(row, t0 + t, part[i]);
+    // Tokens whose x the limbs do not carry (er_nonfinite.h, the conditioning
+    // rule of er_xlimbs.h): their rows again in fp32 from the raw weights, one
+    // row per lane group as the one-token kernels do.
+    for (uint32_t i = tid; i < (nT << lr); i += NT) part[i] = value(i);  // only this thread reads slice 0 of (row, t)
+    __syncthreads();
+    const uint32_t L = o.nfl, G = NT / L, li = lane % L;
+    for (uint32_t i = tid / L; i < (rowsWg + G - 1u) / G * G; i += G) {
+        const uint32_t rw = min(blk * rowsWg + i, M - 1u);
+        for (uint32_t t = 0; t < nT; ++t) {
+            if (!((bad >> t) & 1u)) continue;
+            const bool all = (ill >> t) & 1u;
+            const float *xt = x + (size_t)(t0 + t) * K;
+            float sp[1] = {0.0f}, h = 0.0f;
+            nf_terms<1>([&](int, uint32_t k) { return weight_at<F::FMT>(end.row(rw), k); },
+                        [&](uint32_t k) {
+                            if constexpr (Rows::NORM)
+                                return rows.normW ? xt[k] * rmsv[t] * rows.normW[k] : xt[k];
+                            else
+                                return xt[k];
+                        },
+                        nullptr, K >> 4, li, L, sp, h, all);
+            const float v = tok_group_sum(sp[0], L), hs = tok_group_sum(h, L);
+            if (li == 0 && i < rowsWg && (all || hs > 0.0f)) part[(t << lr) + i] = v;
         }
     }
+    __syncthreads();
+    store_rows([&](uint32_t at) { return part[at]; });
 }
 
 // er_gemv_<fmt>_tok[c|s]_r<RT>_t<4 TG> (W, x, y, M, K, T, order; c, s: MODE), and the fused
