@@ -573,6 +573,202 @@ ER_GEMMP_ENTRY(q8_0, false, 128)
 ER_GEMMP_ENTRY(q8_0, false, 256)
 
 // ---------------------------------------------------------------------------
+// K-grouped variant for shapes whose tiles leave the chip idle: 1024 threads
+// compute a TT x 64 tile of Y (TT tokens), in four groups of 4 waves; group g
+// takes chunks g, g + 4, g + 8, ... of K into two LDS stages of its own, and
+// the groups' accumulators are added through LDS at the end.  So K is split
+// without a zero fill of Y before and atomics into it after.
+//   TT = 32: a group's waves are 2 column blocks x 2 halves of the chunk
+//   TT = 64: 2 token blocks x 2 column blocks
+// Bound: a step's serial chain (barrier, operand reads, products, dequantising,
+// stage writes: 0.75 to 1 us for 256 of K with 4 waves per SIMD). 256 weight
+// rows' lanes read 4 to a row, so the count of loads matters: Q8_0 with its
+// scale as a third load of each lane took 24.7 us at 100x4096x4096, with the
+// scale taken from the neighbouring lanes 17.9 (the split kernel and its zero
+// fill 22.5). Half the groups storing before their products, every guard
+// clamped, was slower (21.0).
+// ---------------------------------------------------------------------------
+// Raw bytes one thread fetches for a quarter of a row's chunk (16 weights).
+// Q4_K: the super-block header and qs bytes [8 q, +8) of the pair: positions
+//       8 q + 0..7 and 32 + 8 q + 0..7.
+//       (e and f)
+// Q8_0: qs bytes [16 (q % 2), +16) of block 2 chunk + q / 2, positions
+//       16 q + 0..15. The chunk's 17 dwords: a holds four, after the middle one
+//       (e: the end of the even block and the odd block's scale) for q > 1; the
+//       even block's qs start 2 bytes into theirs, after its scale.
+struct WQuarter {
+    u32x4 a;
+    uint32_t e, f;
+};
+
+template <bool Q4K>
+ER_DEV void load_wq(const uint8_t *__restrict__ W, uint32_t rowOff, uint32_t chunk, uint32_t q, WQuarter &r) {
+    if (Q4K) {
+        const uint32_t bp = rowOff + (chunk >> 2) * 144u;
+        r.a = ld16_off(W, bp);
+        const uint2 v = *(const uint2 *)(W + (bp + 16u + 32u * (chunk & 3u) + 8u * q));
+        r.e = v.x;
+        r.f = v.y;
+    } else {
+        const uint32_t bp = rowOff + chunk * 68u;
+        r.f = 0;
+        r.a = ld16_off_a4(W, bp + 16u * q + 4u * (q >> 1));
+        r.e = ld4_off(W, bp + 32u);
+    }
+}
+
+template <bool Q4K>
+ER_DEV void dequant_wq(const WQuarter &r, uint32_t chunk, uint32_t q, uint32_t (&out)[8]) {
+    if (Q4K) {
+        const float d = f16_to_f32(r.a.x & 0xffffu), dmin = f16_to_f32(r.a.x >> 16);
+        uint32_t sc2, m2;
+        q4k_scales_pair(r.a.y, r.a.z, r.a.w, chunk & 3u, &sc2, &m2);
+        const float sL = d * ub0(sc2), mL = dmin * ub0(m2);
+        const float sH = d * ub1(sc2), mH = dmin * ub1(m2);
+        const uint32_t qw[2] = {r.e, r.f};
+        const uint32_t M0F = vreg_const(0x0f0f0f0fu);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const uint32_t lo = qw[k] & M0F, hi = (qw[k] >> 4) & M0F;
+            out[2 * k + 0] = pack_bf16x2(__builtin_fmaf(sL, ub0(lo), -mL), __builtin_fmaf(sL, ub1(lo), -mL));
+            out[2 * k + 1] = pack_bf16x2(__builtin_fmaf(sL, ub2(lo), -mL), __builtin_fmaf(sL, ub3(lo), -mL));
+            out[4 + 2 * k + 0] = pack_bf16x2(__builtin_fmaf(sH, ub0(hi), -mH), __builtin_fmaf(sH, ub1(hi), -mH));
+            out[4 + 2 * k + 1] = pack_bf16x2(__builtin_fmaf(sH, ub2(hi), -mH), __builtin_fmaf(sH, ub3(hi), -mH));
+        }
+    } else {
+        const bool odd = q >> 1;
+        // quads of lanes share a row: lane 0's first dword, lane 1's
+        const uint32_t w0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)r.a.x, 0x00, 0xf, 0xf, true);
+        const uint32_t w4 = (uint32_t)__builtin_amdgcn_mov_dpp((int)r.a.x, 0x55, 0xf, 0xf, true);
+        const float d = f16_to_f32(odd ? r.e >> 16 : w0 & 0xffffu);
+        const uint32_t v[5] = {r.a.x, r.a.y, r.a.z, r.a.w, q ? r.e : w4};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t w = odd ? v[k] : alignbyte(v[k + 1], v[k], 2);
+            out[2 * k + 0] = pack_bf16x2(d * sb(w, 0), d * sb(w, 1));
+            out[2 * k + 1] = pack_bf16x2(d * sb(w, 2), d * sb(w, 3));
+        }
+    }
+}
+
+template <bool Q4K, int TT>
+ER_DEV void gemm_q_kg(const uint8_t *__restrict__ W, const uint16_t *__restrict__ X, float *__restrict__ Y,
+                      uint32_t T, uint32_t N, uint32_t K) {
+    constexpr int TN = 64, KG = 4, XL = TT / 32, KS = TT == 32 ? 2 : 4;  // KS: matrix steps per wave and chunk
+    constexpr int ASZ = TT * ER_GEMM_PITCH, BSZ = TN * ER_GEMM_PITCH;
+    constexpr int NP = TT == 32 ? 2 * KG : KG;  // partial tiles
+    extern __shared__ __attribute__((aligned(16))) uint16_t smem[];  // KG x 2 x (A stage + B stage)
+
+    const uint32_t nT = (T + TT - 1) / TT, nN = (N + TN - 1) / TN;
+    const uint32_t total = nT * nN, per = (total + 7u) / 8u, L = blockIdx.x;
+    const uint32_t item = (L % 8u) * per + L / 8u;  // token tile fastest, as in gemm_q_pipe
+    if (item >= total) return;
+    const uint32_t n0 = (item / nT) * TN, t0 = (item % nT) * TT;
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t g = wave >> 2, w = wave & 3u, gt = tid & 255u;
+    uint16_t *base = smem + g * (2u * (ASZ + BSZ));
+    const uint32_t rowBytes = Q4K ? (K >> 8) * 144u : (K >> 6) * 68u;
+    const uint32_t NC = K / ER_GEMM_KC, steps = (NC + KG - 1u) / KG;
+    // W share: row n0 + gt / 4 (clamped), quarter gt % 4; X share: XL 16-byte
+    // pieces, piece i at tile row (gt + 256 i) / 8, k offset 8 ((gt + 256 i) % 8)
+    const uint32_t wq = gt & 3u, wRowOff = min(n0 + (gt >> 2), N - 1u) * rowBytes;
+    uint32_t xOff[XL];
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+        const uint32_t p = gt + 256u * i;
+        xOff[i] = (min(t0 + (p >> 3), T - 1u) * K + 8u * (p & 7u)) * 2u;
+    }
+    WQuarter wr[3];
+    u32x4 xr[3][XL];
+    auto load = [&](uint32_t step, int b) {
+        const uint32_t c = step * KG + g;
+        if (c >= NC) return;  // uniform in the group
+        load_wq<Q4K>(W, wRowOff, c, wq, wr[b]);
+#pragma unroll
+        for (int i = 0; i < XL; ++i) xr[b][i] = ld16_off(X, xOff[i] + c * (ER_GEMM_KC * 2u));
+    };
+    auto store = [&](uint32_t step, int b) {
+        const uint32_t c = step * KG + g;
+        if (c >= NC) return;
+        uint16_t *As = base + (step & 1u) * (ASZ + BSZ), *brow = As + ASZ + (gt >> 2) * ER_GEMM_PITCH;
+        uint32_t wd[8];
+        dequant_wq<Q4K>(wr[b], c, wq, wd);
+        *(u32x4 *)(brow + (Q4K ? 8u * wq : 16u * wq)) = u32x4{wd[0], wd[1], wd[2], wd[3]};
+        *(u32x4 *)(brow + (Q4K ? 32u + 8u * wq : 16u * wq + 8u)) = u32x4{wd[4], wd[5], wd[6], wd[7]};
+#pragma unroll
+        for (int i = 0; i < XL; ++i) {
+            const uint32_t p = gt + 256u * i;
+            *(u32x4 *)(As + (p >> 3) * ER_GEMM_PITCH + 8u * (p & 7u)) = xr[b][i];
+        }
+    };
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    // this wave's block of the tile, and its first matrix step of a chunk
+    const uint32_t nb = w & 1u, tb = TT == 32 ? 0u : w >> 1, k0 = TT == 32 ? w >> 1 : 0u;
+    auto mfma = [&](uint32_t step) {
+        if (step * KG + g >= NC) return;
+        const uint16_t *As = base + (step & 1u) * (ASZ + BSZ);
+        const uint16_t *ap = As + (32u * tb + (lane & 31u)) * ER_GEMM_PITCH + 8u * (lane >> 5) + 32u * k0;
+        const uint16_t *bp = As + ASZ + (32u * nb + (lane & 31u)) * ER_GEMM_PITCH + 8u * (lane >> 5) + 32u * k0;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8 *)(ap + 16 * ks),
+                                                          *(const bf16x8 *)(bp + 16 * ks), acc, 0, 0, 0);
+    };
+    // step s sits in register buffer s % 3; its loads are issued three steps
+    // before its products, one LDS stage is filled while the other is read
+    load(0, 0);
+    load(1, 1);
+    load(2, 2);
+    store(0, 0);
+    for (uint32_t s3 = 0; s3 < steps; s3 += 3u) {
+#pragma unroll
+        for (int B = 0; B < 3; ++B) {
+            const uint32_t s = s3 + (uint32_t)B;
+            if (s >= steps) break;  // uniform
+            __syncthreads();
+            mfma(s);
+            store(s + 1u, (B + 1) % 3);
+            load(s + 3u, B);
+        }
+    }
+    __syncthreads();
+    // partial tiles [NP][TT][64] over the stages; D: col lane % 32, row 8 (r / 4) + 4 (lane / 32) + r % 4
+    float *part = (float *)smem;
+    const uint32_t pi = TT == 32 ? 2u * g + k0 : g;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        part[(pi * TT + 32u * tb + 8u * (r >> 2) + 4u * (lane >> 5) + (r & 3)) * TN + 32u * nb + (lane & 31u)] = acc[r];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TT * TN / 1024; ++i) {
+        const uint32_t o = tid + 1024u * i, t = t0 + o / TN, n = n0 + o % TN;
+        float v[NP];
+#pragma unroll
+        for (int q = 0; q < NP; ++q) v[q] = part[q * (TT * TN) + o];
+#pragma unroll
+        for (int h = NP / 2; h > 0; h /= 2)
+#pragma unroll
+            for (int q = 0; q < h; ++q) v[q] += v[q + h];
+        if (t < T && n < N) Y[(size_t)t * N + n] = v[0];
+    }
+}
+
+#define ER_GEMMK_ENTRY(fmt, q4k, tt)                                                             \
+    extern "C" __global__ void __launch_bounds__(1024)                                         \
+        er_gemmk_##fmt##_t##tt(const uint8_t *__restrict__ W, const uint16_t *__restrict__ X,  \
+                               float *__restrict__ Y, uint32_t T, uint32_t N, uint32_t K) {     \
+        gemm_q_kg<q4k, tt>(W, X, Y, T, N, K);                                                   \
+    }
+
+ER_GEMMK_ENTRY(q4k, true, 32)
+ER_GEMMK_ENTRY(q4k, true, 64)
+ER_GEMMK_ENTRY(q8_0, false, 32)
+ER_GEMMK_ENTRY(q8_0, false, 64)
+
+// ---------------------------------------------------------------------------
 // Loader-specialised variant (512 threads, 128 R weight rows x 128 tokens per
 // workgroup, K % 256 == 0).  Waves 4-5 copy the X tile and waves 6-7 the raw
 // weight bytes of each 64-wide chunk into LDS rings with global_load_lds, each

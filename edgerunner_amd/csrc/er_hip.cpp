@@ -89,6 +89,10 @@ using er_detail::fail;
     X(GEMM_Q8_0_T256, "er_gemm_q8_0_t256")                                             \
     X(GEMMP_Q4K_T64, "er_gemmp_q4k_t64")                                               \
     X(GEMMP_Q8_0_T64, "er_gemmp_q8_0_t64")                                             \
+    X(GEMMK_Q4K_T32, "er_gemmk_q4k_t32")                                               \
+    X(GEMMK_Q4K_T64, "er_gemmk_q4k_t64")                                               \
+    X(GEMMK_Q8_0_T32, "er_gemmk_q8_0_t32")                                             \
+    X(GEMMK_Q8_0_T64, "er_gemmk_q8_0_t64")                                             \
     X(FILL_ZERO, "er_fill_zero")                                                       \
     X(TOP1_REDUCE, "er_top1_reduce")                                                   \
     X(QUANT_Q8_0_V, "er_quantize_q8_0_rows_v")                                         \
@@ -261,7 +265,8 @@ struct er_hip_ctx {
     int cu_mode = -1;      // ER_HIP_GEMV_CU: 0 never, 1 whenever it applies, unset: by shape
     int cuk_mode = -1;     // ER_HIP_GEMV_CUK: 0 never, 2 every K <= 16384, unset: K > 8192 (comparisons)
     int gemm_variant = 0;  // ER_HIP_GEMM_VARIANT=1: non-pipelined GEMM, =2: 256-thread pipelined,
-                           // =3: warp-specialised, =4 / =5: loader-specialised with 256 / 128-row tiles
+                           // =3: warp-specialised, =4 / =5: loader-specialised with 256 / 128-row tiles,
+                           // =6 / =7: K-grouped with 32 / 64-token tiles
                            // wherever it applies (comparisons, tests)
     uint32_t gemm_tt = 0, gemm_sk = 0;  // ER_HIP_GEMM_TILE=tt:sk (benchmark sweeps only)
     int gemv_fp32 = 0;  // ER_HIP_GEMV_FP32=1 selects the fp32 GEMV family (benchmark comparison)
@@ -1107,6 +1112,52 @@ GemmLPlan plan_gemml(const er_hip_ctx *ctx, uint32_t T, uint32_t N, uint32_t K) 
     return p;
 }
 
+// The kernel of a shape whose tiles leave plan_gemml's kernel short of work:
+// returns the token tile of the K-grouped kernel (32 or 64), or 0 with lp set
+// (128-row tiles of the loader-specialised kernel after all) or left alone (the
+// kernels that split K over workgroups: `tiles` tiles, SK splits).
+//
+// Estimates, us, fitted to 60 shapes (16 to 1024 tokens, 1024 to 14336 rows, K
+// 1024 to 4096). K-grouped: 4 chunks of 64 a step, 0.75 us each with 32-token
+// tiles, 0.92 with 64 (1.1 on more than half the CUs, 1.25 over several rounds,
+// where the weights' bandwidth counts). Loader-specialised: 0.43 (Q4_K) or 0.57
+// us a chunk. Split: the zero fill and 0.85 us a chunk, and 2.7 us per million
+// atomics, which is what the K-grouped kernel saves. Measured, us, split ->
+// K-grouped: Q8_0 100x4096x4096 22.5 -> 17.9, 200x2048x2048 17.9 -> 10.2,
+// 64x4096x1024 12.0 -> 6.9, 16x1024x1024 6.3 -> 6.0; Q4_K 100x4096x4096 20.7 ->
+// 17.2, 256x3072x1024 27 -> 8.2, 512x1024x4096 24.1 -> 17.5, 700x1024x4096 30.7
+// -> 20.8. The split keeps few tiles of a long K (Q8_0 32x4096x4096 15.1
+// against 18.6, Q4_K 16x2048x2048 8.0 against 8.9); the loader kernel takes
+// 100x14336x2048 (Q4_K 28.3 split, 24.9 K-grouped, 21.4).
+uint32_t plan_gemmk(const er_hip_ctx *ctx, Fmt f, uint32_t T, uint32_t N, uint32_t K, double tiles, uint32_t SK,
+                    GemmLPlan &lp) {
+    if (ctx->gemm_variant == 6) return 32u;
+    if (ctx->gemm_variant == 7) return 64u;
+    if (ctx->gemm_variant != 0 || ctx->gemm_tt != 0 || ctx->gemm_sk != 0) return 0;
+    const double cu = ctx->cu_count, chunks = K / 64.0, steps = std::ceil(chunks / 4.0);
+    const double cols = (N + 63u) / 64u;
+    double best = SK > 1u ? 4.3 + 0.85 * chunks / SK * std::max(1.0, tiles * SK / cu) + 2.7e-6 * T * N * SK
+                          : 3.0 + 0.85 * chunks * std::max(1.0, tiles / cu);
+    uint32_t tk = 0;
+    for (uint32_t tt : {32u, 64u}) {
+        const double n = cols * ((T + tt - 1u) / tt), rounds = std::ceil(n / cu);
+        const double step = tt == 32u ? 0.75 : rounds > 1.0 ? 1.25 : 2.0 * n > cu ? 1.1 : 0.92;
+        const double cost = 2.5 + rounds * (1.0 + step * steps);
+        if (cost < best && 8u * (tt + 64u) * 144u <= ctx->info.lds_per_workgroup) {
+            best = cost;
+            tk = tt;
+        }
+    }
+    const double n1 = (double)((N + 127u) / 128u) * ((T + 127u) / 128u);
+    const bool fits = K % 256u == 0 && (uint64_t)T * N * 4u < (1ull << 32) && n1 <= 8.0 * 65535.0;
+    if (fits && 3.5 + std::ceil(n1 / cu) * chunks * (f == Fmt::Q4_K ? 0.43 : 0.57) < best) {
+        lp.r = 1;
+        lp.tiles = (uint64_t)n1;
+        return 0;
+    }
+    return tk;
+}
+
 // stamps: null, or (measurement build) 32 bytes per work item for the
 // clock-stamped copy of the kernel
 er_status launch_gemml(er_hip_ctx *ctx, er_stream stream, Fmt f, er_buffer W, er_buffer x, er_buffer y, uint32_t T,
@@ -1164,7 +1215,7 @@ er_status encode_gemm(er_hip_ctx *ctx, er_stream stream, Fmt f, er_buffer W, er_
                     fmt_name(f), (unsigned long long)need, (unsigned long long)T * K * 2u);
     st = bind_device(ctx);
     if (st != ER_OK) return st;
-    const GemmLPlan lp = plan_gemml(ctx, T, N, K);
+    GemmLPlan lp = plan_gemml(ctx, T, N, K);
     if (stamps) {
         if (!lp.r)
             return fail(ER_ERR_INVALID_ARGUMENT, "GEMM clock probe: the loader-specialised kernel does not take "
@@ -1175,16 +1226,29 @@ er_status encode_gemm(er_hip_ctx *ctx, er_stream stream, Fmt f, er_buffer W, er_
         if (stampItems) *stampItems = (uint32_t)lp.tiles;
     }
     if (lp.r) return launch_gemml(ctx, stream, f, W, x, y, T, N, K, lp, stamps ? (uint64_t *)stamps->data : nullptr);
-    // Tile height TT (tokens) and K split SK: 128-token tiles (64 for short
+    // Tile height TT (tokens) and K split SK of the atomics' kernels: 128-token tiles (64 for short
     // inputs), then split K until the grid gives every CU a workgroup
     // (measured on MI355X: 512x14336x4096 is fastest unsplit, 512x4096x4096
     // with two K splits).
     void *args1[] = {&W.data, &x.data, &y.data, &T, &N, &K};
+    const bool atomics = (uint64_t)T * N % 4u == 0 && aligned(y.data, 16);  // as the zero fill needs them
     const uint32_t nN = (N + 127u) / 128u;
     uint32_t TT = T >= 128u ? 128u : 64u, SK = 1u;
     const uint32_t NC = K / 64u;
     while (SK < 8u && 2u * SK <= NC && (uint64_t)nN * ((T + TT - 1u) / TT) * SK < (uint64_t)ctx->cu_count)
         SK *= 2u;
+    const uint32_t tk = plan_gemmk(ctx, f, T, N, K, (double)nN * ((T + TT - 1u) / TT), atomics ? SK : 1u, lp);
+    if (lp.r) return launch_gemml(ctx, stream, f, W, x, y, T, N, K, lp, nullptr);
+    if (tk) {
+        // KG = 4 groups of two stages of (tk + 64) rows of 72 bf16
+        const uint32_t klds = 8u * (tk + 64u) * 144u, kitems = ((N + 63u) / 64u) * ((T + tk - 1u) / tk);
+        if (klds > ctx->info.lds_per_workgroup)
+            return fail(ER_ERR_ENCODING_FAILED, "GEMM: %u B of LDS per workgroup needed, %u available", klds,
+                        (unsigned)ctx->info.lds_per_workgroup);
+        const KernelId kk = f == Fmt::Q4_K ? (tk == 32u ? K_GEMMK_Q4K_T32 : K_GEMMK_Q4K_T64)
+                                           : (tk == 32u ? K_GEMMK_Q8_0_T32 : K_GEMMK_Q8_0_T64);
+        return launch(ctx, kk, dim3(8u * ((kitems + 7u) / 8u), 1, 1), dim3(1024, 1, 1), klds, stream, args1);
+    }
     if (ctx->gemm_tt) TT = ctx->gemm_tt;
     if (ctx->gemm_sk) SK = std::min<uint32_t>(ctx->gemm_sk, NC);
     const uint32_t lds = 2u * (TT + 128u) * 72u * 2u;
@@ -1199,8 +1263,8 @@ er_status encode_gemm(er_hip_ctx *ctx, er_stream stream, Fmt f, er_buffer W, er_
     }
     if (SK > 1u) {
         // split K accumulates with fp32 atomics into a zero-filled Y
-        uint64_t n4 = (uint64_t)T * N / 4u, tail = (uint64_t)T * N % 4u;
-        if (tail || !aligned(y.data, 16)) SK = 1u;
+        uint64_t n4 = (uint64_t)T * N / 4u;
+        if (!atomics) SK = 1u;
         else {
             void *zargs[] = {&y.data, &n4};
             const uint64_t blocks = std::min<uint64_t>((n4 + 255u) / 256u, 4096u);
