@@ -25,7 +25,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 //   Q8_0        5.2 -> 4.8    17.7 -> 13.1    37.2 -> 24.8    58.7 -> 55.8
 // 2048x1024 is level (4.6 us).  A kernel that reads the output right behind
 // the call finds less of it in the caches: the pair is 3-5% slower at
-// 4096x4096, and 4-7% faster for larger K-quant matrices.
+// 4096x4096, and 6-8% faster for larger K-quant matrices.
 ER_DEV void st16_nt(float *p, const float4 &v) {
     __builtin_nontemporal_store(f32x4{v.x, v.y, v.z, v.w}, (f32x4 *)p);
 }
