@@ -90,6 +90,8 @@ ER_DEV bool nf_any_value(const float *v, uint32_t K) {
 // rows whose x the limbs do not carry precisely enough, er_xlimbs.h; with
 // non-finite values present its IEEE sum is the one above, since finite
 // terms cannot cancel an infinite one).
+// The multiply-add is written out: left to the compiler, some kernels fused it
+// and some did not, and a row's last bits differed between them.
 template <int NR, class WAt, class VAt>
 ER_DEV void nf_terms(WAt weight, VAt v, const float *x16, uint32_t C16, uint32_t c0, uint32_t cs,
                      float (&sp)[NR], float &hits, bool all = false) {
@@ -103,7 +105,7 @@ ER_DEV void nf_terms(WAt weight, VAt v, const float *x16, uint32_t C16, uint32_t
             if (!all && __builtin_isfinite(xv)) continue;
             hits += 1.0f;
 #pragma unroll
-            for (int r = 0; r < NR; ++r) sp[r] += __builtin_isnan(xv) ? xv : weight(r, k) * xv;
+            for (int r = 0; r < NR; ++r) sp[r] = __builtin_isnan(xv) ? xv : __builtin_fmaf(weight(r, k), xv, sp[r]);
         }
         bool done = true;
 #pragma unroll
