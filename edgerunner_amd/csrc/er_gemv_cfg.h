@@ -70,6 +70,7 @@ struct TokOrder {
     uint32_t mg;   // i / ns or i / upt of a unit index i as i * mg >> 16
     uint32_t part; // bytes of the partial row sums in LDS
     uint32_t nfl;  // lanes per row of the fp32 re-evaluation
+    uint32_t conv; // how that kernel converts x: bit 0: 8 values a lane (else 16); whole rows: 2 x waves sharing it
 };
 #define ER_TOK_MAX_UNITS 192  // kw * ups: 128 for whole rows (lpr ns / 4), 8 * 9 for K-sliced ones
 // X(RT, TG, 4 TG): 16 RT rows per wave, 4 TG tokens

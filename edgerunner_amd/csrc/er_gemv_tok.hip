@@ -13,8 +13,11 @@
 // Every row value has the bits of the one-token call of the same matrix: the
 // integer sums are exact, each 64-weight slot's contribution is formed by the
 // same fp32 operations, and the slots are added in the order of the one-token
-// kernel that the matrix's M and K select (TokOrder).  So batching tokens
-// never changes a result.
+// kernel that the matrix's M and K select (TokOrder).  Whether a token's rows
+// are evaluated in fp32 instead (the conditioning rule of er_xlimbs.h) is
+// decided as that kernel decides it, from the same pieces of x and, where the
+// order of the sums could matter, in its order.  So batching tokens never
+// changes a result.
 //
 // Work split.  A workgroup of 8 waves owns 16 RT RG rows and 4 TG tokens; RG
 // row groups x KW slices of K (KW RG = 8).  It converts the tokens' x once,
@@ -387,8 +390,9 @@ struct TokOne {
     __device__ __forceinline__ void store(uint32_t r, uint32_t t, float v) const { y[(size_t)t * M + r] = v; }
 };
 // again(): the source for the end of the kernel.  TokQ8Multi (first kernel
-// argument: the Q8Multi block) reads its fields from the argument segment a
-// second time: held over the whole kernel they spilled scalar registers.
+// argument: the Q8Multi block) and TokQ8Pairs (first arguments: TokSiluArgs)
+// read their fields from the argument segment a second time: held over the
+// whole kernel they spilled scalar registers.
 struct TokQ8Multi : CukQ8Multi {
     __device__ __forceinline__ TokQ8Multi(const Q8Multi &mm, size_t rb) : CukQ8Multi(mm, rb) {}
     __device__ __forceinline__ TokQ8Multi again() const {
@@ -408,8 +412,20 @@ struct TokQ8Multi : CukQ8Multi {
     }
     __device__ __forceinline__ void store(uint32_t r, uint32_t t, float v) const { store_at(r, t, v); }
 };
+struct TokSiluArgs {
+    const uint8_t *Wg, *Wu;
+    const float *x;
+    float *y;
+    const float *normW;
+    float eps;
+    uint32_t M;
+};
 struct TokQ8Pairs : CukQ8Pairs {
-    __device__ __forceinline__ const TokQ8Pairs &again() const { return *this; }
+    __device__ __forceinline__ TokQ8Pairs again() const {
+        auto *ka = (const __attribute__((address_space(4))) TokSiluArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(ka));
+        return TokQ8Pairs(CukQ8Pairs{ka->Wg, ka->Wu, ka->y, rowBytes, normW, eps, ka->M});
+    }
     __device__ __forceinline__ TokQ8Pairs(const CukQ8Pairs &p) : CukQ8Pairs(p) {}
     __device__ __forceinline__ void store(uint32_t r, uint32_t t, float v) const { y[(size_t)t * M + (r >> 1)] = v; }
 };
@@ -469,6 +485,55 @@ ER_DEV float tok_sum_sq(const TokOrder &o, const float *__restrict__ x, uint32_t
         for (uint32_t w = 0; w < 4u; ++w) tot += group_sum<64>(ss[w]);
     }
     return tot;
+}
+
+// The conditioning rule as the one-token kernel decides it, its sums added in
+// that kernel's lanes and waves: value16(k, v) gives the 16 values of x from k
+// on as converted, grp holds S float2 of this wave's LDS.  One wave; the result
+// is wave-uniform.  For tokens whose sums lie so near the rule's threshold that
+// the order of the additions could decide (xl_ill_near).
+template <class V>
+ER_DEV bool tok_ill_in_order(const TokOrder &o, uint32_t S, float f, float2 *grp, V value16) {
+    const uint32_t lane = lane_id();
+    const bool half = o.conv & 1u;
+    tok_fence();
+#pragma unroll 1
+    for (uint32_t c0 = 0; c0 < 4u * S; c0 += 64u) {
+        const uint32_t c = c0 + lane;
+        float v[16], ma = 0.0f, mb = 0.0f;
+        value16(16u * min(c, 4u * S - 1u), v);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            ma = fmaxf(ma, fabsf(v[q]));
+            mb = fmaxf(mb, fabsf(v[8 + q]));
+        }
+        float mx = dpp_max_nonneg<ER_DPP_QUAD_XOR1>(fmaxf(ma, mb)), sg, inv;
+        mx = dpp_max_nonneg<ER_DPP_QUAD_XOR2>(mx);
+        xl_scale(mx, &sg, &inv);
+        const float rest = xl_rest_energy16(v, ma, mb, mx, half);
+        if ((c & 3u) == 0u && c < 4u * S) grp[c >> 2] = float2{sg, rest};
+    }
+    tok_fence();
+    const uint32_t ppg = half ? 8u : 4u;  // pieces (lanes) of a 64-group
+    const uint32_t nw = o.ns ? o.conv >> 1 : ER_CU_WAVES, stride = o.ns ? 64u * nw : 64u;
+    float e = 0.0f, r = 0.0f;
+#pragma unroll 1
+    for (uint32_t w = 0; w < nw; ++w) {
+        const uint32_t p0 = o.ns ? 64u * w : ppg * w * o.spw, p1 = ppg * (o.ns ? S : min((w + 1u) * o.spw, S));
+        float ew = 0.0f, rw = 0.0f;
+#pragma unroll 1
+        for (uint32_t p = p0; p < p1; p += stride) {
+            const uint32_t i = p + lane;
+            if (i < p1 && (i & (ppg - 1u)) == 0u) {
+                const float2 g = grp[half ? i >> 3 : i >> 2];
+                ew = __builtin_fmaf(g.y > 0.0f ? g.x : 0.0f, g.x, ew);
+                rw += g.y;
+            }
+        }
+        e += group_sum<64>(ew);
+        r += group_sum<64>(rw);
+    }
+    return xl_ill_rule(e, r, f);
 }
 
 // Rows of the workgroup: RG groups of RT tiles of 16; tokens: 4 TG.  MODE:
@@ -552,6 +617,13 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
     const uint32_t per = o.ns || kw == 1u ? 1u : 8u / kw, nPart = per * kw, stp = TT * rowsWg;
     float *part = (float *)(facs + (kw << o.lupp) * (TT * F::FAC));
     uint32_t nfm = 0;  // tokens with a non-finite chunk sum
+    // x under RMSNorm as converted: whole rows with token t's factor, K-sliced
+    // ones without it (their row values take it)
+    auto normed = [&](const float4 &f, const float4 &w, uint32_t t) {
+        if (!o.ns) return float4{f.x * w.x, f.y * w.y, f.z * w.z, f.w * w.w};
+        const float s = rmsv[t];
+        return float4{f.x * s * w.x, f.y * s * w.y, f.z * s * w.z, f.w * s * w.w};
+    };
     auto convert = [&](uint32_t ps, const float4 (&xr)[4], const float4 (&wr)[NW]) {
         const uint32_t t = ps >> lq, v = 4u * (ps - (t << lq)) + r;
         float xv[16];
@@ -559,15 +631,7 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
         for (int q = 0; q < 4; ++q) {
             float4 f = xr[q];
             if constexpr (Rows::NORM) {
-                if (rows.normW) {
-                    const float4 w = wr[q];
-                    if (o.ns) {
-                        const float s = rmsv[t];
-                        f = float4{f.x * s * w.x, f.y * s * w.y, f.z * s * w.z, f.w * s * w.w};
-                    } else {
-                        f = float4{f.x * w.x, f.y * w.y, f.z * w.z, f.w * w.w};
-                    }
-                }
+                if (rows.normW) f = normed(f, wr[q], t);
             }
             xv[4 * q] = f.x;
             xv[4 * q + 1] = f.y;
@@ -575,7 +639,7 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
             xv[4 * q + 3] = f.w;
         }
         XlChunk ck;
-        xl_chunk(xv, ck);
+        xl_chunk(xv, ck, o.conv & 1u);
         if (__builtin_amdgcn_ballot_w64(!__builtin_isfinite(ck.sum)) != 0) nfm |= 1u << t;
         // the chunk's slot, and the granules of its two 8-value pieces
         constexpr bool Q6 = F::FMT == ER_FMT_Q6_K;
@@ -828,7 +892,6 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
             cu = nu;
         }
     }
-    const Rows end = rows.again();
     // the launch's checks per token
     constexpr uint32_t CW = NT / TT < 64u ? NT / TT : 64u, CN = NT / TT / CW;  // partial sums per token: CN
     ce = group_sum<CW>(ce);
@@ -849,8 +912,30 @@ ER_DEV void gemv_tok(const Rows &rows, const float *__restrict__ x, uint32_t M, 
         ee += c.x;
         rr += c.y;
     }
-    const uint32_t ill = (uint32_t)__builtin_amdgcn_ballot_w64(lane < nT && xl_ill_rule(ee, rr, F::FMT == ER_FMT_Q8_0 ? 1.0f : 4.0f));
+    constexpr float illF = F::FMT == ER_FMT_Q8_0 ? 1.0f : 4.0f;
+    uint32_t ill = (uint32_t)__builtin_amdgcn_ballot_w64(lane < nT && xl_ill_rule(ee, rr, illF));
+    uint32_t near = (uint32_t)__builtin_amdgcn_ballot_w64(lane < nT && xl_ill_near(ee, rr, illF));
+#pragma unroll 1
+    for (; near; near &= near - 1u) {  // alike in every wave
+        const uint32_t t = __builtin_ctz(near);
+        const float *xt = x + (size_t)(t0 + t) * K;
+        const bool b = tok_ill_in_order(o, S, illF, (float2 *)stage, [&](uint32_t k, float (&v)[16]) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float4 f = ((const float4 *)(xt + k))[q];
+                if constexpr (Rows::NORM) {
+                    if (rows.normW) f = normed(f, ((const float4 *)(rows.normW + k))[q], t);
+                }
+                v[4 * q] = f.x;
+                v[4 * q + 1] = f.y;
+                v[4 * q + 2] = f.z;
+                v[4 * q + 3] = f.w;
+            }
+        });
+        ill = b ? ill | 1u << t : ill & ~(1u << t);
+    }
     const uint32_t bad = (uint32_t)__builtin_amdgcn_readfirstlane((int)(ill | nf));
+    const Rows end = rows.again();
     // row value (t, row) at part[t rowsWg + row]: slices as the tree's top
     // levels (whole rows) or in order
     const uint32_t lr = __builtin_ctz(rowsWg);

@@ -648,12 +648,22 @@ TokOrder tok_order_cuk(const CukPlan &kp, Fmt f, uint32_t K) {
         o.upt = std::max(o.upt, (s1 + 3u) / 4u - s0 / 4u);
     }
     o.nfl = 64u / (2u << kp.pi);
+    o.conv = kp.pi == 2 ? 1u : 0u;
     return o;
 }
+// Lane-group kernels: four waves convert x, 16 values a lane.
 TokOrder tok_order_rows(uint32_t lpr, uint32_t ns) {
     TokOrder o{};
     o.lpr = o.nfl = lpr;
     o.ns = ns;
+    o.conv = 2u * ER_GEMV_WAVES;
+    return o;
+}
+// CU-resident kernels: as gemv_cu stages x (STG waves, halfBlocks).
+TokOrder tok_order_cu(const CuCfg &c, uint32_t K) {
+    TokOrder o = tok_order_rows(c.lpr, c.ns);
+    const uint32_t stg = c.ns == 1u || c.ns >= 5u ? ER_CU_WAVES : 4u;
+    o.conv = 2u * stg + (K <= 2048u || (stg == ER_CU_WAVES && K > 8192u) ? 1u : 0u);
     return o;
 }
 bool tok_order(const er_hip_ctx *ctx, Fmt f, uint32_t M, uint32_t K, TokOrder &o) {
@@ -665,7 +675,7 @@ bool tok_order(const er_hip_ctx *ctx, Fmt f, uint32_t M, uint32_t K, TokOrder &o
     CuPlan cp;
     if (plan_cu(ctx, f, M, K, 1u, cp)) {
         const CuCfg &c = (f == Fmt::Q4_K ? kCuCfgQ4K : (f == Fmt::Q8_0 ? kCuCfgQ8 : kCuCfgQ6K))[cp.ci];
-        o = tok_order_rows(c.lpr, c.ns);
+        o = tok_order_cu(c, K);
         return true;
     }
     const int ci = pick_i8(K / 64u, M, ctx->cu_count, 1u);

@@ -80,6 +80,15 @@ ER_DEV XLimbs xl_view(const uint32_t *lds, uint32_t K) {
 // carry energy outside their maximum's lanes, r adds that energy.
 ER_DEV bool xl_ill_rule(float e, float r, float f) { return f * (64.0f / 12.0f) * e > ER_XL_EPS2 * r; }
 
+// Whether the same terms added in another order could decide the rule the
+// other way: at most 256 terms, none negative, so a sum is within 256 * 2^-24
+// = 2^-16 of its exact value, and 2^-14 of r's side covers both sides twice.
+// (Infinite sums count; no terms at all do not.)
+ER_DEV bool xl_ill_near(float e, float r, float f) {
+    const float a = f * (64.0f / 12.0f) * e, b = ER_XL_EPS2 * r;
+    return r > 0.0f && !(fabsf(a - b) > 0x1p-14f * b);
+}
+
 // The launch's end-of-launch checks, gathered while x is converted: each lane
 // adds, over the chunks it converts, the conditioning sums of xl_ill_rule
 // (e: s_g^2 of each group with energy outside its maximum's lanes, r: that
@@ -143,6 +152,21 @@ ER_DEV float xl_group_sum8(float r) {
     return dpp_add<ER_DPP_ROW_HALF_MIRROR>(r);  // quads 2k and 2k+1 of each 8 lanes
 }
 
+// xl_rest_energy for the 4 lanes of a group with 16 values each (maxima ma, mb
+// of a lane's two 8-value halves): a lane holding the group maximum left out
+// whole, or, with `half`, only the half holding it, added as 8 lanes of 8 add.
+ER_DEV float xl_rest_energy16(const float (&v)[16], float ma, float mb, float mx, bool half) {
+    float s1 = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) s1 = __builtin_fmaf(v[q], v[q], s1);
+    float s2 = half ? 0.0f : s1;
+#pragma unroll
+    for (int q = 8; q < 16; ++q) s2 = __builtin_fmaf(v[q], v[q], s2);
+    const bool a = ma == mx, b = mb == mx;
+    const float own = half ? (a ? 0.0f : s1) + (b ? 0.0f : s2) : (a || b ? 0.0f : s2);
+    const float rest = xl_group_sum4(own);
+    return mx > 0.0f && mx < __builtin_inff() ? rest : 0.0f;
+}
 
 // x^2 terms of the RMSNorm sums: one float4's squares, and added to ss.  The
 // fused multiply-adds are written out: left to the compiler, which product of
@@ -186,29 +210,31 @@ ER_DEV void xl_scale(float mx, float *sg, float *inv) {
 // chunk sum, and its 64-group's scale and rest energy.  The 4 chunks of a
 // 64-group are held by 4 consecutive lanes, which exchange their maxima; every
 // lane of the wave must convert together.
+// half: the rest energy of the 8-value halves (xl_store_half), bit for bit, for
+// kernels that share their launch's checks with one that converts in halves.
 struct XlChunk {
     uint32_t lb[ER_XL_PLANES][4];
     float sum, sg, rest;
 };
-ER_DEV void xl_chunk(const float (&v)[16], XlChunk &o) {
-    float mx = 0.0f, sa = 0.0f, sb = 0.0f;
+ER_DEV void xl_chunk(const float (&v)[16], XlChunk &o, bool half = false) {
+    float ma = 0.0f, mb = 0.0f, sa = 0.0f, sb = 0.0f;
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-        mx = fmaxf(mx, fabsf(v[q]));
+        ma = fmaxf(ma, fabsf(v[q]));
         sa += v[q];
     }
 #pragma unroll
     for (int q = 8; q < 16; ++q) {
-        mx = fmaxf(mx, fabsf(v[q]));
+        mb = fmaxf(mb, fabsf(v[q]));
         sb += v[q];
     }
     o.sum = sa + sb;
-    const float lmx = mx;
-    mx = dpp_max_nonneg<ER_DPP_QUAD_XOR1>(mx);
+    const float lmx = fmaxf(ma, mb);
+    float mx = dpp_max_nonneg<ER_DPP_QUAD_XOR1>(lmx);
     mx = dpp_max_nonneg<ER_DPP_QUAD_XOR2>(mx);
     float inv;
     xl_scale(mx, &o.sg, &inv);
-    o.rest = xl_rest_energy(v, lmx, mx, xl_group_sum4);
+    o.rest = xl_rest_energy16(v, ma, mb, mx, half);
     // digits of u = xi + C are bytes 0..2 of fma(v, 1/s_g, 2^23 + C)
     uint32_t u[16];
 #pragma unroll

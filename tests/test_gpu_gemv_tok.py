@@ -96,17 +96,16 @@ def test_every_split(rt, tt):
             c.close()
 
 
-@pytest.mark.parametrize("dim,q,kv,T", [(1024, 70, 30, 5), (2560, 5000, 1300, 3), (4096, 4096, 1024, 18),
-                                        (5120, 300, 77, 6), (14336, 130, 40, 9), (14336, 2100, 40, 2)])
-def test_fused_q8_rows_equal_one_token_calls(tok, dim, q, kv, T):
-    """RMSNorm + QKV (fp32 and fp16 V) and gate/up + SiLU."""
-    ctx = tok
+def check_fused(ctx, dim, q, kv, x, nw):
+    """RMSNorm + QKV (fp32 and fp16 V) and gate/up + SiLU of x [T, dim] against
+    the one-token calls, bit for bit (any NaN equals any other); returns V in
+    fp32 and the activations."""
+    T = len(x)
     f = FusedQ8Kernel(ctx)
     W = [synth.q8_0(synth.seed(97, i), m, dim) for i, m in enumerate((q, kv, kv))]
-    x = synth.normal_f32(synth.seed(97, 5), T * dim)
-    nw = (np.float32(0.5) + np.abs(synth.normal_f32(synth.seed(97, 6), dim))).astype(np.float32)
-    b = [ctx.upload(a) for a in (*W, x, nw)]
+    b = [ctx.upload(a) for a in (*W, np.ascontiguousarray(x), nw)]
     sizes = (4 * q, 4 * kv, 2 * kv, 4 * kv, 4 * kv)  # q, k, v16, v32, act
+    types = (np.float32, np.float32, np.float16, np.float32, np.float32)
     outs = [ctx.alloc(T * n) for n in sizes]
     one = [ctx.alloc(T * n) for n in sizes]
 
@@ -119,11 +118,22 @@ def test_fused_q8_rows_equal_one_token_calls(tok, dim, q, kv, T):
         for t in range(T):
             encode(b[3].view(4 * t * dim, 4 * dim), [o.view(t * n, n) for o, n in zip(one, sizes)], 1)
         ctx.synchronize()
-        for o, w in zip(outs, one):
-            assert np.array_equal(o.download(np.uint8), w.download(np.uint8))
+        got = [o.download(ty).reshape(T, -1) for o, ty in zip(outs, types)]
+        for g, w, ty in zip(got, one, types):
+            assert np.array_equal(g, w.download(ty).reshape(T, -1), equal_nan=True)
+        return got[3], got[4]
     finally:
         for buf in b + outs + one:
             buf.free()
+
+
+@pytest.mark.parametrize("dim,q,kv,T", [(1024, 70, 30, 5), (2560, 5000, 1300, 3), (4096, 4096, 1024, 18),
+                                        (5120, 300, 77, 6), (14336, 130, 40, 9), (14336, 2100, 40, 2)])
+def test_fused_q8_rows_equal_one_token_calls(tok, dim, q, kv, T):
+    """RMSNorm + QKV (fp32 and fp16 V) and gate/up + SiLU."""
+    x = synth.normal_f32(synth.seed(97, 5), T * dim).reshape(T, dim)
+    nw = (np.float32(0.5) + np.abs(synth.normal_f32(synth.seed(97, 6), dim))).astype(np.float32)
+    check_fused(tok, dim, q, kv, x, nw)
 
 
 @pytest.mark.parametrize("M,K", [(100, 1024), (2100, 4096), (60, 14336)])
@@ -140,3 +150,61 @@ def test_x_the_limbs_cannot_carry(tok, fmt, M, K):
     got, one = batched_and_single(tok, fmt, W, x, M, K, T)
     assert np.array_equal(got, one, equal_nan=True)
     assert np.isnan(got[1]).all() and np.isfinite(got[[0, 3, 4, 5]]).all()
+
+
+def _conditioning_x(K, f, half, T):
+    """[T, K] whose tokens step across the rule that sends a call to its fp32
+    evaluation, f (64 / 12) sum s_g^2 > 2^-24 sum rest_g, about 6e-8 of its right
+    side apart: nearer than the order of its fp32 sums matters.  One outlier of
+    1e5 in each 64-group gives every group the scale s_g = 2^-5; rest_g counts the
+    squares outside the outlier's 16 (half: 8) values."""
+    x = synth.normal_f32(synth.seed(99, 1), K).astype(np.float64)
+    rest = x.reshape(-1, 64).copy()
+    rest[:, :8 if half else 16] = 0.0
+    lhs = f * (64.0 / 12.0) * (K / 64.0) * 2.0 ** -10
+    a0 = np.sqrt(lhs / (float(np.float32(5.9604645e-08)) * (rest ** 2).sum()))
+    out = np.empty((T, K), dtype=np.float32)
+    for t in range(T):
+        out[t] = (x * (a0 * (1.0 + (t - T / 2) * 2.0 ** -25))).astype(np.float32)
+        out[t, ::64] = 1e5
+    return out
+
+
+# one-token kernels by how they convert x: 8 values a lane (K-sliced rows of
+# 4096 and less, CU-resident ones of 2048 and less) or 16, in four waves, eight
+# or one slice each
+CONDITIONING = [("q4_k", 2100, 4096, True), ("q4_k", 16400, 1024, True), ("q6_k", 16400, 1024, True),
+                ("q8_0", 5000, 4096, False), ("q4_k", 300, 1024, False), ("q6_k", 1000, 2048, False),
+                ("q8_0", 300, 8192, False), ("q4_k", 260, 14336, False), ("q6_k", 300, 11008, False)]
+
+
+@pytest.mark.parametrize("fmt,M,K,half", CONDITIONING)
+def test_fp32_evaluation_decided_as_the_one_token_call(tok, fmt, M, K, half):
+    """A second outlier beside a group's first, in the same 8 values, in the same
+    16 only and in neither: whether the call falls back to fp32 depends on how
+    its one-token kernel converts x, and batching must not change that; then
+    tokens across the rule's threshold, where the order of its sums decides."""
+    T = 6
+    W = synth.weights(fmt, synth.seed(99, 2), M, K)
+    x = synth.normal_f32(synth.seed(99, 3), T * K).reshape(T, K)
+    x[1:, ::64] = 1e6
+    for t, at in ((2, 7), (3, 8), (4, 15), (5, 16)):
+        x[t, at::64] = 9e5
+    got, one = batched_and_single(tok, fmt, W, x, M, K, T)
+    assert np.array_equal(got, one)
+    x = _conditioning_x(K, 1.0 if fmt == "q8_0" else 4.0, half, 64)
+    got, one = batched_and_single(tok, fmt, W, x, M, K, 64)
+    assert np.array_equal(got, one)
+
+
+@pytest.mark.parametrize("dim", [1024, 4096, 5120])
+def test_fused_fp32_evaluation_decided_as_the_one_token_call(tok, dim):
+    """The same for the fused projections, whose rule sees x under RMSNorm
+    (K-sliced rows: x times the norm weight, here powers of two)."""
+    x = np.concatenate([synth.normal_f32(synth.seed(99, 4), 6 * dim).reshape(6, dim),
+                        _conditioning_x(dim, 1.0, dim == 4096, 64)])
+    x[1:6, ::64] = 1e6
+    for t, at in ((2, 7), (3, 8), (4, 15), (5, 16)):
+        x[t, at::64] = 9e5
+    nw = np.exp2(np.floor(2.0 * np.abs(synth.normal_f32(synth.seed(99, 5), dim // 64)))).astype(np.float32)
+    check_fused(tok, dim, 300, 120, x, np.repeat(nw, 64))
