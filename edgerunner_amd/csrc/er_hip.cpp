@@ -684,12 +684,27 @@ bool tok_order(const er_hip_ctx *ctx, Fmt f, uint32_t M, uint32_t K, TokOrder &o
     return true;
 }
 
+// ER_HIP_GEMV_TOK's value (null: unset).
+void set_tok_mode(er_hip_ctx *ctx, const char *v) {
+    if (!v) return;
+    unsigned a = 0, b = 0, c = 0;
+    if (std::sscanf(v, "%u:%u:%u", &a, &b, &c) == 3) {
+        ctx->tok_mode = 2;
+        ctx->tok_rt = a;
+        ctx->tok_tt = b;
+        ctx->tok_kw = c;
+    } else {
+        ctx->tok_mode = std::atoi(v) != 0 ? 1 : 0;
+    }
+}
+
 // Split of a token-batched launch (er_gemv_tok.hip): configuration {RT, TG}
 // and slices of K kw, for `rows` rows of K weights and T tokens in order o.
 struct TokPlan {
     int ci = -1, mode = 0;
     TokOrder o{};
     uint32_t grid = 0, lds = 0;
+    double cost = 0.0, cost1 = 0.0;  // estimates, us: this launch, the one-token kernels over the tokens
 };
 bool plan_tok(const er_hip_ctx *ctx, int kind, uint32_t rows, uint32_t K, uint32_t T, TokOrder o, TokPlan &p) {
     const bool q6 = kind == TOK_Q6K, q4 = kind == TOK_Q4K;
@@ -699,7 +714,6 @@ bool plan_tok(const er_hip_ctx *ctx, int kind, uint32_t rows, uint32_t K, uint32
     // tokens (Q8_0 and Q6_K with the waits that their larger stages add)
     const double perTile = q4 ? 16.0 : (q6 ? 50.0 : 28.0), perTok = q4 ? 17.0 : (q6 ? 34.0 : 21.0);
     const double rowBytes = (double)K * (q4 ? 0.5625 : (q6 ? 0.8203125 : 1.0625));
-    double best = 0.0;
     for (int ci = 0; ci < kTokCount; ++ci) {
         const TokCfg &c = kTokCfg[ci];
         if (!tok_built(kind, mode, c)) continue;
@@ -731,7 +745,7 @@ bool plan_tok(const er_hip_ctx *ctx, int kind, uint32_t rows, uint32_t K, uint32
             while ((1u << lupp) < t.ups && (uint64_t)(kw << (lupp + 1u)) * unit + fixed <= room) ++lupp;
             t.lupp = lupp;
             const uint32_t blocks = (rows + rowsWg - 1u) / rowsWg;
-            const uint64_t wgs = (uint64_t)blocks * nTok, grid = (uint64_t)((blocks + 7u) / 8u) * 8u * nTok;
+            const uint64_t grid = (uint64_t)((blocks + 7u) / 8u) * 8u * nTok;
             if (grid > 0x7fffffffull) continue;
             // microseconds of a launch, fitted to sweeps over the configurations
             // (14336 x 4096, 4096 x 14336 and 1024 x 1024, 4 to 77 tokens; most
@@ -743,17 +757,24 @@ bool plan_tok(const er_hip_ctx *ctx, int kind, uint32_t rows, uint32_t K, uint32
             // (under RMSNorm the sum of squares and the norm weights as well)
             const bool norm = kind == TOK_Q8_MULTI || kind == TOK_Q8_SILU;
             const double conv = std::min(TT, T) * (K / 1024.0) * (170.0 / 2100.0 + (norm ? 0.2 : 0.0));
-            const double res = c.rt == 1u && wgs > cu ? 2.0 : 1.0;  // workgroups sharing a CU
-            const double rounds = std::ceil((double)wgs / (cu * res));
+            // workgroups of the fullest XCD (row block b on XCD b % 8) over its
+            // CUs, two to a CU where the registers and the LDS allow it: 81
+            // blocks x 3 token tiles are 243 workgroups for 256 CUs, but 33 for
+            // the 32 of XCD 0 (Q8_0 1289 x 6400 x 24 took 36.5 us, the one-token
+            // kernels 19.9)
+            const double perXcd = (double)((blocks + 7u) / 8u) * nTok, cuXcd = cu / 8.0;
+            const uint32_t bytes = (kw << lupp) * unit + fixed;
+            const double res = c.rt == 1u && perXcd > cuXcd && bytes <= ctx->info.lds_per_workgroup / 2u - 4096u ? 2.0 : 1.0;
+            const double rounds = std::ceil(perXcd / (cuXcd * res));
             const double cost = 3.0 + rounds * (1.5 + 0.4 * t.ups + res * (walk + conv + rowsWg * rowBytes / 45000.0));
             if (ctx->tok_mode == 2 && (c.rt != ctx->tok_rt || TT != ctx->tok_tt || kw != ctx->tok_kw)) continue;
-            if (p.ci < 0 || cost < best) {
-                best = cost;
+            if (p.ci < 0 || cost < p.cost) {
+                p.cost = cost;
                 p.ci = ci;
                 p.mode = mode;
                 p.o = t;
                 p.grid = (uint32_t)grid;
-                p.lds = (kw << lupp) * unit + fixed;
+                p.lds = bytes;
             }
         }
     }
@@ -762,7 +783,8 @@ bool plan_tok(const er_hip_ctx *ctx, int kind, uint32_t rows, uint32_t K, uint32
     // Q4_K / Q8_0 / Q6_K 14336 x 4096).  Few tokens and short matrices stay
     // with them.
     const double perTok1 = 0.08 + (double)rows * K * (q4 ? 6.2e-8 : (q6 ? 9.0e-8 : 8.5e-8));
-    if (ctx->tok_mode < 0 && best >= 3.0 + T * perTok1) return false;
+    p.cost1 = 3.0 + T * perTok1;
+    if (ctx->tok_mode < 0 && p.cost >= p.cost1) return false;
     return p.ci >= 0;
 }
 
@@ -1419,6 +1441,20 @@ er_status encode_q4k_geglu(er_hip_ctx *ctx, er_stream stream, er_buffer Wg, er_b
                      stream, args);
 }
 
+// tok_order of the fused Q8_0 projections of `rows` rows (gate and up both).
+bool tok_order_q8_fused(const er_hip_ctx *ctx, uint32_t rows, uint32_t K, bool silu, TokOrder &o) {
+    CukPlan kp;
+    if (fused_on_cuk(ctx, rows, K) && plan_cuk(ctx, Fmt::Q8_0, rows, K, 1u, kp, true)) {
+        o = tok_order_cuk(kp, Fmt::Q8_0, K);
+        return true;
+    }
+    const MultiPick mp = pick_multi(ctx, K / 64u, rows, !silu, 1u);
+    if (mp.ci < 0 && mp.ci1 < 0) return false;
+    const I8Cfg &c = mp.ci >= 0 ? kI8MultiCfg[mp.ci] : kI8Multi1Cfg[mp.ci1];
+    o = tok_order_rows(c.lpr, c.ns);
+    return true;
+}
+
 // Fused Q8_0 projections (Dequant_Q8_0.metal:199-586, encoded by name in
 // LlamaLanguageModel.swift:260-275).  The reference dispatches them without
 // checks; here every buffer must hold what the shapes imply (weights
@@ -1515,19 +1551,7 @@ er_status encode_q8_fused(er_hip_ctx *ctx, er_stream stream, const Q8FusedSpec &
         const int kind = f.silu ? TOK_Q8_SILU : TOK_Q8_MULTI;
         TokOrder o;
         TokPlan tp;
-        bool ok = false;
-        if (fused_on_cuk(ctx, rowsV, K) && plan_cuk(ctx, Fmt::Q8_0, (uint32_t)rowsV, K, 1u, kp, true)) {
-            o = tok_order_cuk(kp, Fmt::Q8_0, K);
-            ok = true;
-        } else {
-            const MultiPick mp = pick_multi(ctx, S, (uint32_t)rowsV, !f.silu, 1u);
-            if (mp.ci >= 0 || mp.ci1 >= 0) {
-                const I8Cfg &c = mp.ci >= 0 ? kI8MultiCfg[mp.ci] : kI8Multi1Cfg[mp.ci1];
-                o = tok_order_rows(c.lpr, c.ns);
-                ok = true;
-            }
-        }
-        if (ok && plan_tok(ctx, kind, (uint32_t)rowsV, K, tokens, o, tp)) {
+        if (tok_order_q8_fused(ctx, (uint32_t)rowsV, K, f.silu, o) && plan_tok(ctx, kind, (uint32_t)rowsV, K, tokens, o, tp)) {
             const dim3 grid(tp.grid, 1, 1), block(64u * ER_CU_WAVES, 1, 1);
             hipFunction_t fn = ctx->fnTok[kind][tp.mode][tp.ci];
             if (f.silu) {
@@ -1825,17 +1849,7 @@ er_status er_hip_create(int device, er_hip_ctx **out_ctx) {
                     return fail(ER_ERR_FUNCTION_NOT_FOUND, "functionNotFound(%s): %s", name, hipGetErrorString(e));
                 }
             }
-    if (const char *tv = std::getenv("ER_HIP_GEMV_TOK")) {
-        unsigned a = 0, b = 0, c = 0;
-        if (std::sscanf(tv, "%u:%u:%u", &a, &b, &c) == 3) {
-            ctx->tok_mode = 2;
-            ctx->tok_rt = a;
-            ctx->tok_tt = b;
-            ctx->tok_kw = c;
-        } else {
-            ctx->tok_mode = std::atoi(tv) != 0 ? 1 : 0;
-        }
-    }
+    set_tok_mode(ctx, std::getenv("ER_HIP_GEMV_TOK"));
     if (const char *gv = std::getenv("ER_HIP_GEMM_VARIANT")) ctx->gemm_variant = std::atoi(gv);
     if (const char *fv = std::getenv("ER_HIP_GEMV_FP32")) ctx->gemv_fp32 = std::atoi(fv);
     if (const char *gt = std::getenv("ER_HIP_GEMM_TILE")) {
@@ -2386,6 +2400,30 @@ er_status er_hip_encode_projection(er_hip_ctx *ctx, er_stream stream,
 
 #ifdef ER_WITH_PROBES
 // ---- measurement kernels (er_hip_probe.h; the measurement library only) ----
+
+er_status er_hip_probe_tok_plan(uint32_t kind, uint32_t rows, uint32_t K, uint32_t tokens, uint32_t cu_count,
+                                const char *mode, uint32_t *plan, float *cost) {
+    if (kind >= (uint32_t)TOK_KINDS || !plan || !cost || cu_count < 8u)
+        return fail(ER_ERR_INVALID_ARGUMENT, "token plan probe: kind %u, %u CUs", kind, cu_count);
+    er_hip_ctx ctx;
+    ctx.cu_count = (int)cu_count;
+    ctx.info.lds_per_workgroup = 163840u;
+    set_tok_mode(&ctx, mode);
+    const Fmt f = kind == TOK_Q4K ? Fmt::Q4_K : (kind == TOK_Q6K ? Fmt::Q6_K : Fmt::Q8_0);
+    TokOrder o;
+    TokPlan p;
+    const bool fused = kind == TOK_Q8_MULTI || kind == TOK_Q8_SILU;
+    const bool taken = tok_applies(&ctx, K, tokens) &&
+                       (fused ? tok_order_q8_fused(&ctx, rows, K, kind == TOK_Q8_SILU, o) : tok_order(&ctx, f, rows, K, o)) &&
+                       plan_tok(&ctx, (int)kind, rows, K, tokens, o, p);
+    std::memset(plan, 0, 8u * sizeof(uint32_t));
+    cost[0] = (float)p.cost;
+    cost[1] = (float)p.cost1;
+    if (!taken) return ER_OK;
+    const uint32_t v[8] = {1u, kTokCfg[p.ci].rt, 4u * kTokCfg[p.ci].tg, p.o.kw, (uint32_t)p.mode, p.grid, p.lds, 1u << p.o.lupp};
+    std::memcpy(plan, v, sizeof(v));
+    return ER_OK;
+}
 
 // One workgroup per CU for the per-CU rate probes: 96 KB of LDS each, so no
 // second workgroup fits beside it.

@@ -35,6 +35,16 @@ er_status er_hip_probe_stream_read(er_hip_ctx *ctx, er_stream stream, er_buffer 
 er_status er_hip_probe_gemm_clock(er_hip_ctx *ctx, er_stream stream, er_tensor_type type, er_buffer weight,
                                   er_buffer x_bf16, er_buffer y, uint32_t tokens, uint32_t N, uint32_t K,
                                   er_buffer stamps, uint32_t *items);
+/* The launch that a call of `tokens` tokens takes on a card of cu_count compute
+ * units (160 KiB of LDS each); needs no device.  kind 0 Q4_K, 1 Q8_0, 2 Q6_K
+ * matrices of `rows` rows, 3 the fused Q8_0 rows (all matrices'), 4 the fused
+ * gate/up pairs (both matrices' rows); mode as ER_HIP_GEMV_TOK, or null.
+ * plan[8]: 1 if the token-batched kernels take it (else all 0), row tiles per
+ * wave, tokens per workgroup, slices of K, addition mode (0 one slot per leaf,
+ * 1 several, 2 slices inside a unit), workgroups, LDS bytes, units per phase.
+ * cost[2]: the estimates compared, us: the best split, the one-token kernels. */
+er_status er_hip_probe_tok_plan(uint32_t kind, uint32_t rows, uint32_t K, uint32_t tokens, uint32_t cu_count,
+                                const char *mode, uint32_t *plan, float *cost);
 /* One launch of an empty 64-thread kernel. */
 er_status er_hip_probe_empty(er_hip_ctx *ctx, er_stream stream);
 /* `rounds` grid-wide barriers across `workgroups` single-wave workgroups
