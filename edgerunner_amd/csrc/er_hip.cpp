@@ -781,9 +781,13 @@ bool plan_tok(const er_hip_ctx *ctx, int kind, uint32_t rows, uint32_t K, uint32
     // the one-token kernels over the tokens: a launch, then every token's
     // weights again (from the Infinity Cache: 3.2 / 7.3 / 4.4 us per token of
     // Q4_K / Q8_0 / Q6_K 14336 x 4096).  Few tokens and short matrices stay
-    // with them.
+    // with them.  Below 768 rows their tokens share the card and cost less than
+    // that, while a batched launch is mostly the conversion of x: of 3594 random
+    // calls with both sides within a factor of two, 43 that the batched kernels
+    // took were slower there by more than 3% (Q4_K 289 x 1024 x 48 9.3 us
+    // against 7.4), with the 0.85 19 are.
     const double perTok1 = 0.08 + (double)rows * K * (q4 ? 6.2e-8 : (q6 ? 9.0e-8 : 8.5e-8));
-    p.cost1 = 3.0 + T * perTok1;
+    p.cost1 = (3.0 + T * perTok1) * (rows < 768u ? 0.85 : 1.0);
     if (ctx->tok_mode < 0 && p.cost >= p.cost1) return false;
     return p.ci >= 0;
 }
