@@ -714,6 +714,35 @@ bool plan_tok(const er_hip_ctx *ctx, int kind, uint32_t rows, uint32_t K, uint32
     // tokens (Q8_0 and Q6_K with the waits that their larger stages add)
     const double perTile = q4 ? 16.0 : (q6 ? 50.0 : 28.0), perTok = q4 ? 17.0 : (q6 ? 34.0 : 21.0);
     const double rowBytes = (double)K * (q4 ? 0.5625 : (q6 ? 0.8203125 : 1.0625));
+    // the one-token kernels over the tokens: a launch, then every token's
+    // weights again (from the Infinity Cache: 3.2 / 7.3 / 4.4 us per token of
+    // Q4_K / Q8_0 / Q6_K 14336 x 4096).  Few tokens and short matrices stay
+    // with them.
+    const double perTok1 = 0.08 + (double)rows * K * (q4 ? 6.2e-8 : (q6 ? 9.0e-8 : 8.5e-8));
+    const bool norm = kind == TOK_Q8_MULTI || kind == TOK_Q8_SILU;
+    p.cost1 = 3.0 + T * perTok1;
+    if (rows < 768u && !norm) {
+        // Matrices this short stay in the L2s, and a token costs its slots, the
+        // row's idle lanes with them (lane groups, K-sliced), while a batched
+        // launch is mostly the conversion of x.  Less a tenth, the estimates'
+        // error: of 3594 random calls with both sides within a factor of two the
+        // batched kernels lost more than 3% in 43 (Q4_K 289 x 1024 x 48 9.3 us
+        // against 7.4), with this in 28.
+        const double slot = o.ns ? (q6 ? 0.110 : 0.073) : (q4 ? 0.058 : (q6 ? 0.087 : 0.063));
+        const double lanes = o.ns ? o.lpr * o.ns : 8u * o.nfl;
+        p.cost1 = std::min(p.cost1, 0.9 * (3.2 + rows * rowBytes * 1e-7 + T * (4e-6 * K + slot * rows * lanes * 64e-6)));
+    }
+    // microseconds of a launch, fitted to sweeps over the configurations
+    // (14336 x 4096, 4096 x 14336 and 1024 x 1024, 4 to 77 tokens; most
+    // within 15%): vector time at 2.1 GHz of a workgroup's walk (two
+    // waves per SIMD) and of its conversion of x (a pass of 170
+    // instructions per 1024 values; under RMSNorm the sum of squares and the
+    // norm weights as well), a latency per unit, the weight bytes, and a start
+    // per workgroup and launch
+    const auto walk_us = [&](uint32_t units, uint32_t rt, uint32_t tg) {
+        return units * 4.0 * rt * (perTile + perTok * tg) * 8.0 / 2100.0;
+    };
+    const auto conv_us = [&](uint32_t TT) { return std::min(TT, T) * (K / 1024.0) * (170.0 / 2100.0 + (norm ? 0.2 : 0.0)); };
     for (int ci = 0; ci < kTokCount; ++ci) {
         const TokCfg &c = kTokCfg[ci];
         if (!tok_built(kind, mode, c)) continue;
@@ -747,26 +776,19 @@ bool plan_tok(const er_hip_ctx *ctx, int kind, uint32_t rows, uint32_t K, uint32
             const uint32_t blocks = (rows + rowsWg - 1u) / rowsWg;
             const uint64_t grid = (uint64_t)((blocks + 7u) / 8u) * 8u * nTok;
             if (grid > 0x7fffffffull) continue;
-            // microseconds of a launch, fitted to sweeps over the configurations
-            // (14336 x 4096, 4096 x 14336 and 1024 x 1024, 4 to 77 tokens; most
-            // within 15%): vector time at 2.1 GHz of a workgroup's walk (two
-            // waves per SIMD) and of its conversion of x (a pass of 170
-            // instructions per 1024 values), a latency per unit, the weight
-            // bytes, and a start per workgroup and launch
-            const double walk = t.ups * 4.0 * c.rt * (perTile + perTok * c.tg) * 8.0 / 2100.0;
-            // (under RMSNorm the sum of squares and the norm weights as well)
-            const bool norm = kind == TOK_Q8_MULTI || kind == TOK_Q8_SILU;
-            const double conv = std::min(TT, T) * (K / 1024.0) * (170.0 / 2100.0 + (norm ? 0.2 : 0.0));
             // workgroups of the fullest XCD (row block b on XCD b % 8) over its
-            // CUs, two to a CU where the registers and the LDS allow it: 81
-            // blocks x 3 token tiles are 243 workgroups for 256 CUs, but 33 for
-            // the 32 of XCD 0 (Q8_0 1289 x 6400 x 24 took 36.5 us, the one-token
-            // kernels 19.9)
+            // CUs: 81 blocks x 3 token tiles are 243 workgroups for 256 CUs, but
+            // 33 for the 32 of XCD 0 (Q8_0 1289 x 6400 x 24 took 36.5 us, the
+            // one-token kernels 19.9).  With one row tile a second workgroup on
+            // a CU counts as a full round's work without its latency, whether
+            // the two fit side by side or not; where the LDS holds one, counting
+            // single rounds instead favoured splits of many workgroups (Q8_0
+            // 4096 x 14336 x 77 picked 198 us over 154)
             const double perXcd = (double)((blocks + 7u) / 8u) * nTok, cuXcd = cu / 8.0;
-            const uint32_t bytes = (kw << lupp) * unit + fixed;
-            const double res = c.rt == 1u && perXcd > cuXcd && bytes <= ctx->info.lds_per_workgroup / 2u - 4096u ? 2.0 : 1.0;
+            const double res = c.rt == 1u && perXcd > cuXcd ? 2.0 : 1.0;
             const double rounds = std::ceil(perXcd / (cuXcd * res));
-            const double cost = 3.0 + rounds * (1.5 + 0.4 * t.ups + res * (walk + conv + rowsWg * rowBytes / 45000.0));
+            const double cost = 3.0 + rounds * (1.5 + 0.4 * t.ups + res * (walk_us(t.ups, c.rt, c.tg) + conv_us(TT) +
+                                                                         rowsWg * rowBytes / 45000.0));
             if (ctx->tok_mode == 2 && (c.rt != ctx->tok_rt || TT != ctx->tok_tt || kw != ctx->tok_kw)) continue;
             if (p.ci < 0 || cost < p.cost) {
                 p.cost = cost;
@@ -774,20 +796,10 @@ bool plan_tok(const er_hip_ctx *ctx, int kind, uint32_t rows, uint32_t K, uint32
                 p.mode = mode;
                 p.o = t;
                 p.grid = (uint32_t)grid;
-                p.lds = bytes;
+                p.lds = (kw << lupp) * unit + fixed;
             }
         }
     }
-    // the one-token kernels over the tokens: a launch, then every token's
-    // weights again (from the Infinity Cache: 3.2 / 7.3 / 4.4 us per token of
-    // Q4_K / Q8_0 / Q6_K 14336 x 4096).  Few tokens and short matrices stay
-    // with them.  Below 768 rows their tokens share the card and cost less than
-    // that, while a batched launch is mostly the conversion of x: of 3594 random
-    // calls with both sides within a factor of two, 43 that the batched kernels
-    // took were slower there by more than 3% (Q4_K 289 x 1024 x 48 9.3 us
-    // against 7.4), with the 0.85 19 are.
-    const double perTok1 = 0.08 + (double)rows * K * (q4 ? 6.2e-8 : (q6 ? 9.0e-8 : 8.5e-8));
-    p.cost1 = (3.0 + T * perTok1) * (rows < 768u ? 0.85 : 1.0);
     if (ctx->tok_mode < 0 && p.cost >= p.cost1) return false;
     return p.ci >= 0;
 }
