@@ -743,6 +743,10 @@ bool plan_tok(const er_hip_ctx *ctx, int kind, uint32_t rows, uint32_t K, uint32
         return units * 4.0 * rt * (perTile + perTok * tg) * 8.0 / 2100.0;
     };
     const auto conv_us = [&](uint32_t TT) { return std::min(TT, T) * (K / 1024.0) * (170.0 / 2100.0 + (norm ? 0.2 : 0.0)); };
+    // no split beats one round of one unit of the smallest: where that loses
+    // already, the search is not made (0.25 us of the host's 3 per call, which a
+    // plain loop of small calls ran at)
+    if (ctx->tok_mode < 0 && 3.0 + 1.5 + 0.4 + walk_us(1, 1, 1) + conv_us(4) >= p.cost1) return false;
     for (int ci = 0; ci < kTokCount; ++ci) {
         const TokCfg &c = kTokCfg[ci];
         if (!tok_built(kind, mode, c)) continue;

@@ -48,6 +48,21 @@ def test_short_matrices(kind, rows, K, T, taken):
     assert (plan(kind, rows, K, T)[0] is not None) == taken
 
 
+def test_taken_exactly_where_the_estimate_says():
+    """The bound that turns small calls away before the search decides no call
+    otherwise than the search does."""
+    rng = random.Random(6)
+    taken = 0
+    for _ in range(4000):
+        kind, T = rng.choice(list(KINDS)), int(2 ** rng.uniform(1, 7))
+        rows, K = int(2 ** rng.uniform(6, 14)), 256 * int(2 ** rng.uniform(0, 6))
+        best, one = plan(kind, rows, K, T, "1")[1]
+        got = plan(kind, rows, K, T)[0]
+        assert (got is not None) == (best < one), (kind, rows, K, T, best, one)
+        taken += got is not None
+    assert 500 < taken < 3500
+
+
 def test_launches_are_the_kernels():
     """Whatever the shape: a built split, as many workgroups as its grid mapping
     needs, LDS within the CU's."""
