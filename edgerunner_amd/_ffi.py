@@ -214,6 +214,7 @@ PROBE_SIGNATURES = {
     "er_hip_probe_stream_read": (C.c_int, [_ctx_p, _stream, er_buffer, _u64, _u32, er_buffer]),
     "er_hip_probe_tok_plan": (C.c_int, [_u32, _u32, _u32, _u32, _u32, C.c_char_p, C.POINTER(C.c_uint32),
                                         C.POINTER(C.c_float)]),
+    "er_hip_probe_gemm_plan": (C.c_int, [C.c_int, _u32, _u32, _u32, _u32, C.POINTER(C.c_uint32)]),
     "er_hip_probe_empty": (C.c_int, [_ctx_p, _stream]),
     "er_hip_probe_grid_barrier": (C.c_int, [_ctx_p, _stream, _u32, _u32, _u32, er_buffer, er_buffer]),
     "er_hip_probe_lds_read": (C.c_int, [_ctx_p, _stream, _u32, _u32, er_buffer]),

@@ -1169,18 +1169,21 @@ GemmLPlan plan_gemml(const er_hip_ctx *ctx, uint32_t T, uint32_t N, uint32_t K) 
 // (128-row tiles of the loader-specialised kernel after all) or left alone (the
 // kernels that split K over workgroups: `tiles` tiles, SK splits).
 //
-// Estimates, us, fitted to 60 shapes (16 to 1024 tokens, 1024 to 14336 rows, K
-// 1024 to 4096). K-grouped: 4 chunks of 64 a step, 0.75 us each with 32-token
-// tiles, 0.92 with 64 (1.1 on more than half the CUs, 1.25 over several rounds,
-// where the weights' bandwidth counts). Loader-specialised: 0.43 (Q4_K) or 0.57
-// us a chunk. Split: the zero fill and 0.85 us a chunk, and 2.7 us per million
-// atomics, which is what the K-grouped kernel saves. Measured, us, split ->
-// K-grouped: Q8_0 100x4096x4096 22.5 -> 17.9, 200x2048x2048 17.9 -> 10.2,
-// 64x4096x1024 12.0 -> 6.9, 16x1024x1024 6.3 -> 6.0; Q4_K 100x4096x4096 20.7 ->
-// 17.2, 256x3072x1024 27 -> 8.2, 512x1024x4096 24.1 -> 17.5, 700x1024x4096 30.7
-// -> 20.8. The split keeps few tiles of a long K (Q8_0 32x4096x4096 15.1
-// against 18.6, Q4_K 16x2048x2048 8.0 against 8.9); the loader kernel takes
-// 100x14336x2048 (Q4_K 28.3 split, 24.9 K-grouped, 21.4).
+// Estimates, us, fitted to 250 random shapes in both formats with every kernel
+// timed (2 to 2048 tokens, 256 to 20000 rows, K 256 to 14336, fewer tiles than
+// the loader kernel's bound); the choice is 0.4% off the fastest on average and
+// behind the split by more than 3% in 1 of 500.  K-grouped: a round of
+// workgroups starts, then 4 chunks of 64 a step, longer by the weight bytes of a
+// step over the chip and by how full it is.  Loader-specialised: a chunk, longer
+// by its weight bytes.  Split: the zero fill, 0.58 us a chunk (1.05, with
+// 128-token tiles 1.2, once the splits outnumber the CUs and two share one), and
+// 2.7 us per million atomics, which is what the K-grouped kernel saves.  Measured, us, split -> K-grouped: Q8_0 100x4096x4096
+// 21.9 -> 17.1, 200x2048x2048 17.3 -> 9.5, 64x4096x1024 12.0 -> 6.8, 11x264x768
+// 7.0 -> 4.9; Q4_K 100x4096x4096 20.5 -> 17.1, 256x3072x1024 26.8 -> 7.8,
+// 512x1024x4096 23.6 -> 16.0, 700x1024x4096 29.8 -> 18.8.  The split keeps few
+// tiles of a long K (Q4_K 13x6192x4608 16.8 against 18.5, 10x6456x6656 19.7
+// against 24.2); the loader kernel takes 100x14336x2048 (Q4_K 26.8 split, 24.9
+// K-grouped, 20.4).
 uint32_t plan_gemmk(const er_hip_ctx *ctx, Fmt f, uint32_t T, uint32_t N, uint32_t K, double tiles, uint32_t SK,
                     GemmLPlan &lp) {
     if (ctx->gemm_variant == 6) return 32u;
@@ -1188,13 +1191,15 @@ uint32_t plan_gemmk(const er_hip_ctx *ctx, Fmt f, uint32_t T, uint32_t N, uint32
     if (ctx->gemm_variant != 0 || ctx->gemm_tt != 0 || ctx->gemm_sk != 0) return 0;
     const double cu = ctx->cu_count, chunks = K / 64.0, steps = std::ceil(chunks / 4.0);
     const double cols = (N + 63u) / 64u;
-    double best = SK > 1u ? 4.3 + 0.85 * chunks / SK * std::max(1.0, tiles * SK / cu) + 2.7e-6 * T * N * SK
+    double best = SK > 1u ? 4.8 + chunks / SK * (tiles * SK <= cu ? 0.58 : T < 128u ? 1.05 : 1.2) + 2.7e-6 * T * N * SK
                           : 3.0 + 0.85 * chunks * std::max(1.0, tiles / cu);
+    // MB of weights in a step of a round: 64 rows a column, 4 chunks
+    const double stepMB = std::min(cols, cu) * 64.0 * 256.0 * (f == Fmt::Q4_K ? 0.5625e-6 : 1.0625e-6);
     uint32_t tk = 0;
     for (uint32_t tt : {32u, 64u}) {
-        const double n = cols * ((T + tt - 1u) / tt), rounds = std::ceil(n / cu);
-        const double step = tt == 32u ? 0.75 : rounds > 1.0 ? 1.25 : 2.0 * n > cu ? 1.1 : 0.92;
-        const double cost = 2.5 + rounds * (1.0 + step * steps);
+        const double n = cols * ((T + tt - 1u) / tt), rounds = std::ceil(n / cu), full = n / rounds / cu;
+        const double cost = tt == 32u ? 2.0 + rounds * (1.25 + (0.67 + 0.06 * stepMB + 0.11 * full) * steps)
+                                      : 1.0 + rounds * (2.2 + (0.84 + 0.035 * stepMB + 0.18 * full) * steps);
         if (cost < best && 8u * (tt + 64u) * 144u <= ctx->info.lds_per_workgroup) {
             best = cost;
             tk = tt;
@@ -1202,12 +1207,39 @@ uint32_t plan_gemmk(const er_hip_ctx *ctx, Fmt f, uint32_t T, uint32_t N, uint32
     }
     const double n1 = (double)((N + 127u) / 128u) * ((T + 127u) / 128u);
     const bool fits = K % 256u == 0 && (uint64_t)T * N * 4u < (1ull << 32) && n1 <= 8.0 * 65535.0;
-    if (fits && 3.5 + std::ceil(n1 / cu) * chunks * (f == Fmt::Q4_K ? 0.43 : 0.57) < best) {
+    // ... of a chunk in the loader kernel: 128 rows a column
+    const double chunkMB = (N + 127u) / 128u * 128.0 * 64.0 * (f == Fmt::Q4_K ? 0.5625e-6 : 1.0625e-6);
+    if (fits && 3.5 + std::ceil(n1 / cu) * chunks * ((f == Fmt::Q4_K ? 0.42 : 0.455) + 0.2 * chunkMB) < best) {
         lp.r = 1;
         lp.tiles = (uint64_t)n1;
         return 0;
     }
     return tk;
+}
+
+// What a GEMM call launches: the loader-specialised kernel (lp.r != 0), the
+// K-grouped kernel with token tiles of tk, or tiles of TT tokens with SK splits
+// of K, added with atomics where SK > 1 (`atomics`: Y takes the zero fill).
+struct GemmPlan {
+    GemmLPlan lp;
+    uint32_t tk = 0, TT = 0, SK = 1;
+};
+// Tile height and K split of the atomics' kernels: 128-token tiles (64 for short
+// inputs), then split K until the grid gives every CU a workgroup (measured on
+// MI355X: 512x14336x4096 is fastest unsplit, 512x4096x4096 with two K splits).
+GemmPlan plan_gemm(const er_hip_ctx *ctx, Fmt f, uint32_t T, uint32_t N, uint32_t K, bool atomics) {
+    GemmPlan p;
+    p.lp = plan_gemml(ctx, T, N, K);
+    if (p.lp.r) return p;
+    const uint32_t nN = (N + 127u) / 128u, NC = K / 64u;
+    p.TT = T >= 128u ? 128u : 64u;
+    const uint64_t tiles = (uint64_t)nN * ((T + p.TT - 1u) / p.TT);
+    while (p.SK < 8u && 2u * p.SK <= NC && tiles * p.SK < (uint64_t)ctx->cu_count) p.SK *= 2u;
+    p.tk = plan_gemmk(ctx, f, T, N, K, (double)tiles, atomics ? p.SK : 1u, p.lp);
+    if (ctx->gemm_tt) p.TT = ctx->gemm_tt;
+    if (ctx->gemm_sk) p.SK = std::min<uint32_t>(ctx->gemm_sk, NC);
+    if (!atomics) p.SK = 1u;
+    return p;
 }
 
 // stamps: null, or (measurement build) 32 bytes per work item for the
@@ -1267,7 +1299,9 @@ er_status encode_gemm(er_hip_ctx *ctx, er_stream stream, Fmt f, er_buffer W, er_
                     fmt_name(f), (unsigned long long)need, (unsigned long long)T * K * 2u);
     st = bind_device(ctx);
     if (st != ER_OK) return st;
-    GemmLPlan lp = plan_gemml(ctx, T, N, K);
+    const bool atomics = (uint64_t)T * N % 4u == 0 && aligned(y.data, 16);  // as the zero fill needs them
+    const GemmPlan gp = plan_gemm(ctx, f, T, N, K, atomics);
+    const GemmLPlan &lp = gp.lp;
     if (stamps) {
         if (!lp.r)
             return fail(ER_ERR_INVALID_ARGUMENT, "GEMM clock probe: the loader-specialised kernel does not take "
@@ -1278,19 +1312,9 @@ er_status encode_gemm(er_hip_ctx *ctx, er_stream stream, Fmt f, er_buffer W, er_
         if (stampItems) *stampItems = (uint32_t)lp.tiles;
     }
     if (lp.r) return launch_gemml(ctx, stream, f, W, x, y, T, N, K, lp, stamps ? (uint64_t *)stamps->data : nullptr);
-    // Tile height TT (tokens) and K split SK of the atomics' kernels: 128-token tiles (64 for short
-    // inputs), then split K until the grid gives every CU a workgroup
-    // (measured on MI355X: 512x14336x4096 is fastest unsplit, 512x4096x4096
-    // with two K splits).
     void *args1[] = {&W.data, &x.data, &y.data, &T, &N, &K};
-    const bool atomics = (uint64_t)T * N % 4u == 0 && aligned(y.data, 16);  // as the zero fill needs them
-    const uint32_t nN = (N + 127u) / 128u;
-    uint32_t TT = T >= 128u ? 128u : 64u, SK = 1u;
-    const uint32_t NC = K / 64u;
-    while (SK < 8u && 2u * SK <= NC && (uint64_t)nN * ((T + TT - 1u) / TT) * SK < (uint64_t)ctx->cu_count)
-        SK *= 2u;
-    const uint32_t tk = plan_gemmk(ctx, f, T, N, K, (double)nN * ((T + TT - 1u) / TT), atomics ? SK : 1u, lp);
-    if (lp.r) return launch_gemml(ctx, stream, f, W, x, y, T, N, K, lp, nullptr);
+    const uint32_t nN = (N + 127u) / 128u, NC = K / 64u, tk = gp.tk, TT = gp.TT;
+    uint32_t SK = gp.SK;
     if (tk) {
         // KG = 4 groups of two stages of (tk + 64) rows of 72 bf16
         const uint32_t klds = 8u * (tk + 64u) * 144u, kitems = ((N + 63u) / 64u) * ((T + tk - 1u) / tk);
@@ -1301,8 +1325,6 @@ er_status encode_gemm(er_hip_ctx *ctx, er_stream stream, Fmt f, er_buffer W, er_
                                            : (tk == 32u ? K_GEMMK_Q8_0_T32 : K_GEMMK_Q8_0_T64);
         return launch(ctx, kk, dim3(8u * ((kitems + 7u) / 8u), 1, 1), dim3(1024, 1, 1), klds, stream, args1);
     }
-    if (ctx->gemm_tt) TT = ctx->gemm_tt;
-    if (ctx->gemm_sk) SK = std::min<uint32_t>(ctx->gemm_sk, NC);
     const uint32_t lds = 2u * (TT + 128u) * 72u * 2u;
     if (ctx->gemm_variant == 1 || lds > ctx->info.lds_per_workgroup) {
         // single-stage kernel (benchmark comparison, or two LDS stages do not fit)
@@ -1316,13 +1338,10 @@ er_status encode_gemm(er_hip_ctx *ctx, er_stream stream, Fmt f, er_buffer W, er_
     if (SK > 1u) {
         // split K accumulates with fp32 atomics into a zero-filled Y
         uint64_t n4 = (uint64_t)T * N / 4u;
-        if (!atomics) SK = 1u;
-        else {
-            void *zargs[] = {&y.data, &n4};
-            const uint64_t blocks = std::min<uint64_t>((n4 + 255u) / 256u, 4096u);
-            st = launch(ctx, K_FILL_ZERO, dim3((uint32_t)blocks, 1, 1), dim3(256, 1, 1), 0, stream, zargs);
-            if (st != ER_OK) return st;
-        }
+        void *zargs[] = {&y.data, &n4};
+        const uint64_t blocks = std::min<uint64_t>((n4 + 255u) / 256u, 4096u);
+        st = launch(ctx, K_FILL_ZERO, dim3((uint32_t)blocks, 1, 1), dim3(256, 1, 1), 0, stream, zargs);
+        if (st != ER_OK) return st;
     }
     KernelId k;
     if (TT == 256u) k = f == Fmt::Q4_K ? K_GEMMP_Q4K_T256 : K_GEMMP_Q8_0_T256;
@@ -2442,6 +2461,21 @@ er_status er_hip_probe_tok_plan(uint32_t kind, uint32_t rows, uint32_t K, uint32
     if (!taken) return ER_OK;
     const uint32_t v[8] = {1u, kTokCfg[p.ci].rt, 4u * kTokCfg[p.ci].tg, p.o.kw, (uint32_t)p.mode, p.grid, p.lds, 1u << p.o.lupp};
     std::memcpy(plan, v, sizeof(v));
+    return ER_OK;
+}
+
+er_status er_hip_probe_gemm_plan(er_tensor_type type, uint32_t tokens, uint32_t N, uint32_t K, uint32_t cu_count,
+                                 uint32_t *plan) {
+    if ((type != ER_TYPE_Q4_K && type != ER_TYPE_Q8_0) || !plan || cu_count == 0 || tokens == 0 || N == 0 || K == 0)
+        return fail(ER_ERR_INVALID_ARGUMENT, "GEMM plan probe: tokens %u, N %u, K %u", tokens, N, K);
+    er_hip_ctx ctx;
+    ctx.cu_count = (int)cu_count;
+    ctx.info.lds_per_workgroup = 163840u;
+    const GemmPlan p = plan_gemm(&ctx, type == ER_TYPE_Q4_K ? Fmt::Q4_K : Fmt::Q8_0, tokens, N, K,
+                                 (uint64_t)tokens * N % 4u == 0);
+    plan[0] = p.lp.r ? (uint32_t)p.lp.r : (p.tk ? 3u : 0u);
+    plan[1] = p.lp.r ? 128u : (p.tk ? p.tk : p.TT);
+    plan[2] = p.lp.r || p.tk ? 1u : p.SK;
     return ER_OK;
 }
 

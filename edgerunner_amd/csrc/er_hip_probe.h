@@ -45,6 +45,12 @@ er_status er_hip_probe_gemm_clock(er_hip_ctx *ctx, er_stream stream, er_tensor_t
  * cost[2]: the estimates compared, us: the best split, the one-token kernels. */
 er_status er_hip_probe_tok_plan(uint32_t kind, uint32_t rows, uint32_t K, uint32_t tokens, uint32_t cu_count,
                                 const char *mode, uint32_t *plan, float *cost);
+/* What a GEMM call (Y 16-byte aligned) launches on a card of cu_count compute
+ * units; needs no device.  plan[3]: 1 or 2 the loader-specialised kernel with
+ * 128- or 256-row tiles, 3 the K-grouped kernel, 0 the others; tokens per tile;
+ * splits of K over workgroups. */
+er_status er_hip_probe_gemm_plan(er_tensor_type type, uint32_t tokens, uint32_t N, uint32_t K, uint32_t cu_count,
+                                 uint32_t *plan);
 /* One launch of an empty 64-thread kernel. */
 er_status er_hip_probe_empty(er_hip_ctx *ctx, er_stream stream);
 /* `rounds` grid-wide barriers across `workgroups` single-wave workgroups

@@ -2,8 +2,8 @@
 (ER_HIP_GEMM_VARIANT=6: 32 tokens, 7: 64) where it can go wrong: one token and
 one past a tile, one row and one past a tile, K of one chunk (three of the four
 groups have none), of five and seven chunks (a last step that not all groups
-have) and of whole steps; then the shapes that select it unforced against the
-kernels that split K over workgroups.  Bars: 1e-5 against the float64 product
+have) and of whole steps; then shapes that select it unforced, by their bits,
+against the kernels that split K over workgroups.  Bars: 1e-5 against the float64 product
 with the bf16-rounded weights, fp32 sums of at most 2048 products being within
 2048 * 2^-24 = 1.2e-4 of the sum of magnitudes at the worst and about its
 square root, 3e-6, as they come; two kernels are twice that apart."""
@@ -41,14 +41,18 @@ def test_forced(variant, fmt, T, N, K):
 
 
 @pytest.mark.parametrize("fmt", ["q4_k", "q8_0"])
-@pytest.mark.parametrize("T,N,K", [(16, 1024, 1024), (100, 2048, 1024), (129, 1031, 512), (257, 3072, 1024), (100, 14336, 256)])
-def test_selected_against_the_split(fmt, T, N, K):
+@pytest.mark.parametrize("T,N,K,tile", [(16, 1024, 1024, 32), (100, 2048, 1024, 32), (128, 1032, 512, 32),
+                                        (257, 3072, 1024, 64), (60, 14336, 256, 64)])
+def test_selected_against_the_split(fmt, T, N, K, tile):
+    assert T * N % 4 == 0  # else the forced split would not split
     W, X = _case(fmt, T, N, K)
     out = []
-    for env in ({}, {"ER_HIP_GEMM_TILE": "64:4"}):
+    for env in ({}, {"ER_HIP_GEMM_VARIANT": "6" if tile == 32 else "7"}, {"ER_HIP_GEMM_TILE": "64:4"}):
         c, gemm = _gemm(**env)
         try:
             out.append(gemm.execute(fmt, W, X, T, N, K))
         finally:
             c.close()
-    assert rel_l2(out[0], out[1]) < 2e-5
+    # the sums of the K-grouped kernel in its own order: it is the one that ran
+    assert np.array_equal(out[0], out[1]) and not np.array_equal(out[0], out[2])
+    assert rel_l2(out[0], out[2]) < 2e-5
