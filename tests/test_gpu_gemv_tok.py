@@ -5,6 +5,7 @@ K-sliced rows whose slices start at and inside a 256-weight unit), row and
 token remainders, every compiled configuration and slice count, and x the
 limbs cannot carry.  The one-token calls are themselves held to the oracle
 (test_gpu_gemv.py, test_gpu_gemv_cuk.py, test_gpu_fused_q8.py)."""
+import functools
 import os
 
 import numpy as np
@@ -14,6 +15,7 @@ import edgerunner_amd.synth as synth
 from edgerunner_amd import Context, FusedQ8Kernel, GEMVKernel
 from oracle import ref
 from conftest import rel_l2
+from test_tok_plan import plan
 
 pytestmark = pytest.mark.gpu
 
@@ -70,30 +72,102 @@ SHAPES = [(1, 256, 2), (17, 512, 3), (33, 1280, 9), (300, 1024, 5), (9000, 768, 
 def test_rows_equal_one_token_calls(tok, fmt, M, K, T):
     W = synth.weights(fmt, synth.seed(96, 1), M, K)
     x = synth.normal_f32(synth.seed(96, 2), T * K)
+    x[K:2 * K] = -0.0  # a token of nothing: its rows keep the one-token call's zeros, sign and all
     got, one = batched_and_single(tok, fmt, W, x, M, K, T)
-    assert np.array_equal(got, one)
+    assert np.array_equal(got.view(np.uint32), one.view(np.uint32))
     rows = slice(0, min(M, 64))
     n = len(W) // M
     exp = np.stack([ref.gemv(fmt, W[:n * min(M, 64)], x[t * K:(t + 1) * K], min(M, 64), K) for t in (0, T - 1)])
     assert rel_l2(got[[0, T - 1]][:, rows], exp) < 1e-3
 
 
-@pytest.mark.parametrize("rt,tt", [(1, 4), (4, 4), (1, 8), (4, 8), (1, 16), (2, 16)])
-def test_every_split(rt, tt):
-    """Each compiled {row tiles, tokens} with every count of K slices, plain
-    rows (K = 1024), chained slots (9000 x 768), split slices (K = 5120) and
-    several phases (K = 14336)."""
+SPLITS = [(1, 4), (4, 4), (1, 8), (4, 8), (1, 16), (2, 16)]  # {row tiles, tokens}, with 1, 2, 4 or 8 slices of K
+PLAIN, CHAINED, INSIDE = range(3)  # one slot per leaf, several, slices that start inside a unit
+
+
+def reached(kind):
+    """The (addition mode, row tiles, tokens, slices) that some shape can take:
+    compiled, with enough leaves for the slices, and within the LDS."""
+    few = {(PLAIN, 2, 16, 8)} if kind != "q4_k" else set()
+    small = kind not in ("q4_k", "q8_0")  # chained slots of these: as INSIDE of Q8_0, without {4, 8}
+    out = set()
+    for rt, tt in SPLITS:
+        for kw in (1, 2, 4, 8):
+            out.add((PLAIN, rt, tt, kw))
+            if kw == 1 or small:  # whole rows of Q4_K and Q8_0 chain on four lanes only
+                out.add((CHAINED, rt, tt, kw))
+            if kind != "q6_k":
+                out.add((INSIDE, rt, tt, kw))
+    if small:
+        few |= {(CHAINED, 4, 8, kw) for kw in (1, 2, 4, 8)} | {(CHAINED, 2, 16, 8)}
+    if kind not in ("q4_k", "q6_k"):
+        few |= {(INSIDE, 4, 8, kw) for kw in (1, 2, 4, 8)} | {(INSIDE, 2, 16, 2), (INSIDE, 2, 16, 8)}
+    return out - few
+
+
+@functools.lru_cache(maxsize=None)
+def split_case(fmt, M, K, T):
+    return synth.weights(fmt, synth.seed(96, 3), M, K), synth.normal_f32(synth.seed(96, 4), T * K)
+
+
+SPLIT_SHAPES = {"q4_k": [(70, 1024, 5), (9000, 512, 2), (9000, 256, 2), (50, 5120, 6), (45, 14336, 18)],
+                "q8_0": [(70, 1024, 5), (9000, 512, 2), (9000, 256, 2), (50, 4352, 6), (45, 14336, 18)],
+                "q6_k": [(40, 256, 5), (9000, 256, 2), (9000, 512, 5), (16500, 4352, 3), (45, 14336, 18), (8300, 12544, 2)]}
+
+
+@pytest.mark.parametrize("rt,tt", SPLITS)
+@pytest.mark.parametrize("fmt", FMTS)
+def test_every_split(fmt, rt, tt):
+    """Every compiled {row tiles, tokens} with every count of K slices that a
+    shape can take, in each addition mode and over one and several phases.  A
+    split that a shape does not take is left out: the call would run the
+    one-token kernels."""
+    ran = set()
     for kw in (1, 2, 4, 8):
-        c = forced(f"{rt}:{tt}:{kw}")
+        split = f"{rt}:{tt}:{kw}"
+        c = forced(split)
         try:
-            for M, K, T in ((70, 1024, 5), (9000, 768, 2), (50, 5120, 6), (45, 14336, 18)):
-                for fmt in FMTS:
-                    W = synth.weights(fmt, synth.seed(96, 3), M, K)
-                    x = synth.normal_f32(synth.seed(96, 4), T * K)
-                    got, one = batched_and_single(c, fmt, W, x, M, K, T)
-                    assert np.array_equal(got, one), (kw, M, K, T, fmt)
+            assert c.compute_units == 256
+            for M, K, T in SPLIT_SHAPES[fmt]:
+                p, _ = plan(fmt, M, K, T, split)
+                if p is None:
+                    continue
+                assert p[:3] == (rt, tt, kw)
+                got, one = batched_and_single(c, fmt, *split_case(fmt, M, K, T), M, K, T)
+                assert np.array_equal(got, one), (kw, M, K, T, fmt)
+                ran.add((p[3], rt, tt, kw))
         finally:
             c.close()
+    assert ran == {r for r in reached(fmt) if r[1:3] == (rt, tt)}
+
+
+@pytest.mark.parametrize("rt,tt", SPLITS)
+def test_every_split_fused(rt, tt):
+    """The same for the fused projections' rows and gate/up pairs."""
+    ran = {"q8_rows": set(), "q8_pairs": set()}
+    for kw in (1, 2, 4, 8):
+        split = f"{rt}:{tt}:{kw}"
+        c = forced(split)
+        try:
+            for q, kv, dim in ((40, 20, 256), (40, 20, 4352), (5000, 4500, 512), (4000, 4500, 256), (4000, 4500, 2304),
+                               (4000, 4500, 6912), (45, 20, 14336)):
+                taken = {k: plan(k, n, dim, 5, split)[0] for k, n in (("q8_rows", q + 2 * kv), ("q8_pairs", 2 * kv))}
+                if not any(taken.values()):
+                    continue
+                x = synth.normal_f32(synth.seed(97, 7), 5 * dim).reshape(5, dim)
+                check_fused(c, dim, q, kv, x, np.abs(synth.normal_f32(synth.seed(97, 8), dim)))
+                for k, p in taken.items():
+                    if p is not None:
+                        ran[k].add((p[3], rt, tt, kw))
+        finally:
+            c.close()
+    for k, r in ran.items():
+        assert r == {w for w in reached(k) if w[1:3] == (rt, tt)}, k
+
+
+@functools.lru_cache(maxsize=None)
+def fused_weights(q, kv, dim):
+    return [synth.q8_0(synth.seed(97, i), m, dim) for i, m in enumerate((q, kv, kv))]
 
 
 def check_fused(ctx, dim, q, kv, x, nw):
@@ -102,7 +176,7 @@ def check_fused(ctx, dim, q, kv, x, nw):
     fp32 and the activations."""
     T = len(x)
     f = FusedQ8Kernel(ctx)
-    W = [synth.q8_0(synth.seed(97, i), m, dim) for i, m in enumerate((q, kv, kv))]
+    W = fused_weights(q, kv, dim)
     b = [ctx.upload(a) for a in (*W, np.ascontiguousarray(x), nw)]
     sizes = (4 * q, 4 * kv, 2 * kv, 4 * kv, 4 * kv)  # q, k, v16, v32, act
     types = (np.float32, np.float32, np.float16, np.float32, np.float32)
@@ -134,6 +208,25 @@ def test_fused_q8_rows_equal_one_token_calls(tok, dim, q, kv, T):
     x = synth.normal_f32(synth.seed(97, 5), T * dim).reshape(T, dim)
     nw = (np.float32(0.5) + np.abs(synth.normal_f32(synth.seed(97, 6), dim))).astype(np.float32)
     check_fused(tok, dim, q, kv, x, nw)
+
+
+@pytest.mark.parametrize("dim,q,kv", [(1024, 70, 30), (2560, 5000, 1300), (4096, 4096, 1024), (5120, 300, 77),
+                                      (14336, 130, 40)])
+def test_fused_x_the_limbs_cannot_carry(tok, dim, q, kv):
+    """Tokens with NaN, with infinities, with outliers that send the call to its
+    fp32 evaluation, and with a NaN and outliers, under RMSNorm: rows of every
+    matrix and gate/up pairs equal the one-token calls bit for bit."""
+    assert plan("q8_rows", q + 2 * kv, dim, 8, "1")[0] and plan("q8_pairs", 2 * kv, dim, 8, "1")[0]
+    x = synth.normal_f32(synth.seed(97, 9), 8 * dim).reshape(8, dim)
+    x[1, 5] = np.nan
+    x[2, dim - 1], x[2, 70] = np.inf, -np.inf
+    x[3, 64] = np.inf
+    x[5, ::64] = 1e6
+    x[6, ::64], x[6, dim - 2] = 1e6, np.nan
+    nw = (np.float32(0.5) + np.abs(synth.normal_f32(synth.seed(97, 10), dim))).astype(np.float32)
+    v, act = check_fused(tok, dim, q, kv, x, nw)
+    for y in (v, act):
+        assert np.isnan(y[[1, 6]]).all() and np.isfinite(y[[0, 4, 5, 7]]).all() and not np.isfinite(y[[2, 3]]).any()
 
 
 @pytest.mark.parametrize("M,K", [(100, 1024), (2100, 4096), (60, 14336)])
