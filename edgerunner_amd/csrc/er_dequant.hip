@@ -17,15 +17,21 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Stores past the caches.  The kernels are bound by their 4 bytes out per
 // weight, which they never read again; stored the ordinary way those lines are
-// kept in L2 and displace each other and the blocks still to be read.
-// Measured over rotating outputs, us a call, ordinary -> these (same card):
-//               2049x2048      4096x4096       8192x4096       14336x4096
-//   Q4_K        5.4 -> 4.6    15.5 -> 11.9    27.6 -> 22.1    50.5 -> 38.6
-//   Q6_K        5.4 -> 4.7    16.6 -> 12.5    30.6 -> 23.9    50.6 -> 40.6
-//   Q8_0        5.2 -> 4.8    17.7 -> 13.1    37.2 -> 24.8    58.7 -> 55.8
-// 2048x1024 is level (4.6 us).  A kernel that reads the output right behind
-// the call finds less of it in the caches: the pair is 3-5% slower at
-// 4096x4096, and 6-8% faster for larger K-quant matrices.
+// kept in L2 and the Infinity Cache and displace each other and the blocks still
+// to be read.  Measured us a call, ordinary -> these, on one card, every call
+// with blocks and an output that no call before it touched for over 1 GB, as
+// matrices are widened once at load:
+//               2049x2048     4096x4096      8192x4096      14336x4096     28672x8192
+//   Q4_K        5.8 -> 4.3   15.5 -> 13.9   27.6 -> 25.8   50.5 -> 47.6   230 -> 226
+//   Q6_K        5.8 -> 4.2   16.6 -> 15.7   30.5 -> 28.7   51.0 -> 49.4   215 -> 208
+//   Q8_0        6.4 -> 5.3   17.8 -> 16.8   37.4 -> 34.9   57.2 -> 53.9   225 -> 218
+// 1024x1024 is level (3.7 us).  With the same blocks in every call they gain
+// more (14336x4096 Q6_K 50.6 -> 40.6: the blocks then stay cached).  What they
+// cost: an output buffer written again and again no longer stays in the Infinity
+// Cache (fresh blocks into one buffer: 4096x4096 15.3 -> 15.7, 14336x4096 Q4_K
+// 44.8 -> 47.6, Q8_0 50.3 -> 53.8), and a kernel that reads the output right
+// behind the call finds less of it in the caches (the pair: 4096x4096 5-8%
+// slower, 8192x4096 level to 5% faster, beyond that level to 5% faster).
 ER_DEV void st16_nt(float *p, const float4 &v) {
     __builtin_nontemporal_store(f32x4{v.x, v.y, v.z, v.w}, (f32x4 *)p);
 }

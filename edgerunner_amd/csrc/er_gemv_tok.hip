@@ -28,20 +28,22 @@
 // 16), so the four limb sums of a (row, token) are one lane's registers and
 // the rescaling needs no cross-lane step.
 //
-// Bound: vector instructions.  Per 64-weight slot a (16 rows x 4 tokens) tile
+// Bound: vector instructions, and the waits of one or two waves per SIMD for
+// LDS reads and each other.  Per 64-weight slot a (16 rows x 4 tokens) tile
 // costs about 17 of them (Q4_K; Q8_0 15, Q6_K 30) plus 14 (8, 38) per row tile
 // for the quants and scales, against 2 (2, 4) matrix instructions (taking those
 // out changes no time); the conversion of x costs as much as 1.5 row tiles (of
 // 16 tokens) per workgroup, which is why the rows of a workgroup go up with
-// the launch (plan_tok).  Counters of 14336 x 4096 Q4_K x 77 tokens: the vector
-// units busy 72% of the time the CUs are, and 560 workgroups on 256 CUs leave
-// the last of three rounds a fifth full.
-// Measured, us a call, the one-token kernels over the tokens -> these (the
-// planner's choice; weights of several matrices in turn):
+// the launch (plan_tok).  Counters of 77 tokens: the vector units busy 63% of
+// the time the CUs are (Q4_K 14336 x 4096; Q8_0 49%, with the LDS active 52%;
+// Q6_K 4096 x 14336 63%), the matrix cores 13 to 22%, and 1120 workgroups on
+// 256 CUs leave the last of five rounds three eighths full (Q4_K, Q8_0).
+// Measured, us a call in a graph, the one-token kernels over the tokens ->
+// these (the planner's choice; weights of several matrices in turn, 600 MB):
 //   tokens            5             16             32             77
-//   Q4_K 14336x4096   25.8 -> 18.9   57.5 -> 33.3  111.0 -> 47.4  254.6 -> 112
-//   Q8_0 14336x4096   39.9 -> 26.4  117.7 -> 36.0  233.8 -> 50.4  559.7 -> 136
-//   Q6_K 4096x14336   40.3 -> 36.8  102.2 -> 58.0  201.7 -> 90.1  482.5 -> 228
+//   Q4_K 14336x4096   25.4 -> 18.2   51.0 -> 31.6   97.8 -> 44.8  232 -> 133
+//   Q8_0 14336x4096   40.3 -> 26.5  120 -> 36.4    237 -> 51.0    565 -> 147
+//   Q6_K 4096x14336   40.4 -> 36.6  103 -> 57.7    201 -> 89.7    482 -> 228
 #include "er_gemv_cfg.h"
 
 // One wave-uniform unit of work: super-block sb (256 weights) of the slice.
