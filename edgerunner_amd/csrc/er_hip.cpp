@@ -725,16 +725,17 @@ bool plan_tok(const er_hip_ctx *ctx, int kind, uint32_t rows, uint32_t K, uint32
         // Matrices this short stay in the L2s, and a token costs its slots, the
         // row's idle lanes with them (lane groups, K-sliced), while a batched
         // launch is mostly the conversion of x.  Less a tenth, the estimates'
-        // error: of 3594 random calls with both sides within a factor of two the
-        // batched kernels lost more than 3% in 43 (Q4_K 289 x 1024 x 48 9.3 us
-        // against 7.4), with this in 28.
+        // error.  Of 2511 random calls that the batched kernels take 66 were more
+        // than 3% slower there (Q4_K 289 x 1024 x 48 9.3 us against 7.4), with
+        // this and the rounds by XCD below 46.
         const double slot = o.ns ? (q6 ? 0.110 : 0.073) : (q4 ? 0.058 : (q6 ? 0.087 : 0.063));
         const double lanes = o.ns ? o.lpr * o.ns : 8u * o.nfl;
         p.cost1 = std::min(p.cost1, 0.9 * (3.2 + rows * rowBytes * 1e-7 + T * (4e-6 * K + slot * rows * lanes * 64e-6)));
     }
     // microseconds of a launch, fitted to sweeps over the configurations
-    // (14336 x 4096, 4096 x 14336 and 1024 x 1024, 4 to 77 tokens; most
-    // within 15%): vector time at 2.1 GHz of a workgroup's walk (two
+    // (14336 x 4096, 4096 x 14336 and 1024 x 1024, 4 to 77 tokens; over 690
+    // other matrices most within 15%, slices that start inside a unit and the
+    // fused forms up to 30% low): vector time at 2.1 GHz of a workgroup's walk (two
     // waves per SIMD) and of its conversion of x (a pass of 170
     // instructions per 1024 values; under RMSNorm the sum of squares and the
     // norm weights as well), a latency per unit, the weight bytes, and a start
